@@ -53,9 +53,11 @@ typedef enum {
     VKBLAS_KERNEL_PIPE256 = 3,          /* pipelined kernel, 256 x 256 tiles       */
     VKBLAS_KERNEL_PIPE128 = 4,          /* pipelined kernel, 128 x 128, 2 stages   */
     VKBLAS_KERNEL_PIPE128_4 = 5,        /* pipelined kernel, 128 x 128, 4 stages   */
-    VKBLAS_KERNEL_SKINNY = 6,           /* decode kernels                          */
-    VKBLAS_KERNEL_WAVEK = 7             /* split-K pass 1 on 32 x 32 / 64 x 64
+    VKBLAS_KERNEL_SKINNY = 6,           /* decode plans (vkblas_last_path skinny)  */
+    VKBLAS_KERNEL_WAVEK = 7,            /* split-K pass 1 on 32 x 32 / 64 x 64
                                            tiles, the slice's K over the waves  */
+    VKBLAS_KERNEL_DIRECT = 8            /* small tiles, K over the waves, MFMA
+                                           fragments straight from memory       */
 } vkblas_kernel_t;
 
 typedef struct {

@@ -1,0 +1,85 @@
+"""gemm_direct_kernel (small tiles, fragments straight from memory) at the
+edges of its tiles: one past and one short of a tile, one k, K around its K
+step (16 fp32, 32 16-bit) and around a whole round of loads in flight, every
+layout and type pair, odd leading dimensions with NaN in the padding,
+operands one element off any alignment, batches, beta with C in place or
+apart, a bias; against the CPU oracle.  C's padding must come back untouched."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+CONV = {"f32": lambda x: x, "f16": oracle.f2h_rne, "bf16": oracle.f2bf_rne}
+BACK = {"f32": lambda x: x, "f16": oracle.h2f, "bf16": oracle.bf2f}
+TD = {"f32": torch.float32, "f16": torch.float16, "bf16": torch.bfloat16}
+TYPES = [("f32", "f32"), ("f32", "f16"), ("f32", "bf16"), ("f16", "f16"), ("f16", "f32"), ("bf16", "bf16"),
+         ("bf16", "f32")]
+# M, N, K, batch.  64 x 64 tiles from 144 of them on, else 32 x 32 (fp32 with
+# fewer than 128 of those: 16 x 32)
+SHAPES = [(33, 32, 1, 1), (65, 47, 15, 1), (95, 33, 33, 2), (129, 65, 64, 3),   # 16 x 32 (fp32) / 32 x 32
+          (193, 191, 129, 4),                                                   # 32 x 32
+          (65, 64, 257, 72), (129, 127, 511, 36), (193, 321, 1027, 7)]           # 64 x 64
+
+
+def _dev(a, dt):
+    t = torch.from_numpy(a.view(np.int16) if a.dtype == np.uint16 else a).to("cuda:0")
+    return t.view(TD[dt]) if dt != "f32" else t
+
+
+@pytest.mark.parametrize("form", ["plain", "apart"])
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("op_a,op_b", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("ab,ct", TYPES)
+def test_direct(ab, ct, op_a, op_b, shape, form):
+    import vkblas_amd as vk
+    from gpu_helpers import normwise, f32_bound, F16_BOUND, BF16_BOUND
+    M, N, K, batch = shape
+    print(f"[case] direct {ab}>{ct} op={op_a}{op_b} {shape} {form}", flush=True)
+    r = np.random.default_rng(M + 3 * N + 7 * K + batch)
+    # odd leading dimensions, every matrix one element off its buffer's start
+    ra, ca = (K, M) if op_a else (M, K)
+    rb, cb = (N, K) if op_b else (K, N)
+    lda, ldb, ldc = ca + 1 - ca % 2 + 2, cb + 1 - cb % 2 + 4, N + 1 - N % 2 + 2
+    sa, sb, sc = lda * ra + 1, ldb * rb + 3, ldc * M + 5
+
+    def operand(rows, cols, ld, stride):
+        x = np.full(1 + stride * batch, np.nan, np.float32)
+        for i in range(batch):
+            x[1 + i * stride:][:ld * rows].reshape(rows, ld)[:, :cols] = r.uniform(-1, 1, (rows, cols))
+        return x
+    a, b = CONV[ab](operand(ra, ca, lda, sa)), CONV[ab](operand(rb, cb, ldb, sb))
+    c0 = CONV[ct](r.uniform(-1, 1, 1 + sc * batch).astype(np.float32))
+    cin = CONV[ct](r.uniform(-1, 1, 1 + sc * batch).astype(np.float32))
+    bias = CONV[ab](r.uniform(-1, 1, N).astype(np.float32))
+    alpha, beta = 1.25, 0.0 if form == "plain" else -0.5
+    if form == "plain":                  # beta == 0 never reads C
+        for i in range(batch):
+            c0[1 + i * sc:][:ldc * M].reshape(M, ldc)[:, :N] = CONV[ct](np.full(1, np.nan, np.float32))[0]
+    want = c0.copy()
+    for i in range(batch):
+        src = (cin if form == "apart" else want)[1 + i * sc:][:ldc * M].copy()
+        out = want[1 + i * sc:][:ldc * M].copy()
+        oracle.ref_gemm_epi_rm(ab, ct, op_a, op_b, M, N, K, np.ascontiguousarray(a[1 + i * sa:][:lda * ra]), lda,
+                               np.ascontiguousarray(b[1 + i * sb:][:ldb * rb]), ldb, alpha, beta, src, ldc, out, ldc,
+                               BACK[ab](bias))
+        want[1 + i * sc:][:ldc * M] = out
+    dt = {"f32": vk.DT_F32, "f16": vk.DT_F16, "bf16": vk.DT_BF16}
+    dA, dB, dC, dI, dBias = _dev(a, ab), _dev(b, ab), _dev(c0, ct), _dev(cin, ct), _dev(bias, ab)
+    ea, ec = dA.element_size(), dC.element_size()
+    vk.gemm_ex_async(dt[ab], dt[ct], op_a, op_b, M, N, K, alpha, dA.data_ptr() + ea, lda, dB.data_ptr() + ea, ldb,
+                     beta, dC.data_ptr() + ec, ldc, batch=batch, stride_a=sa, stride_b=sb, stride_c=sc,
+                     c_in=dI.data_ptr() + ec if form == "apart" else None, ldc_in=ldc if form == "apart" else 0,
+                     stride_c_in=sc if form == "apart" else 0, bias=dBias.data_ptr(), bias_type=dt[ab])
+    torch.cuda.synchronize()
+    assert vk.last_kernel() == vk.KERNEL_DIRECT, vk.last_kernel()
+    got = dC.cpu().view(torch.int16).numpy().view(np.uint16) if ct != "f32" else dC.cpu().numpy()
+    bound = BF16_BOUND if ct == "bf16" else F16_BOUND if "f16" in (ab, ct) or ab == "bf16" else f32_bound(K)
+    for i in range(batch):
+        g = BACK[ct](got[1 + i * sc:][:ldc * M]).reshape(M, ldc)
+        w = BACK[ct](want[1 + i * sc:][:ldc * M]).reshape(M, ldc)
+        assert np.array_equal(g[:, N:], w[:, N:]), "C padding written"
+        assert np.all(np.isfinite(g[:, :N]))
+        assert normwise(g[:, :N], w[:, :N]) <= bound, i

@@ -694,6 +694,23 @@ static void prof_end(prof_t* pf, hipStream_t stream, const char* what, int ok) {
     hipEventDestroy(pf->e1);
 }
 
+/* A decode-planned call small enough for gemm_direct_kernel, one launch of
+ * small tiles: the decode kernels then run a handful of workgroups, or split
+ * K and pay a second launch for the reduce.  Measured (us, decode kernels
+ * against direct, one box; calls under 8.2 us are bound by the launch):
+ *   fp32 NT, 64 rows: 128 x 256 9.5 / 8.1, 1024^2 13.6 / 10.1; 512 x 4096
+ *   14.4 / 22.1, 2048^2 15.3 / 24.1; NN, 1-64 rows: 1024^2 11.2-13.9 / 8.2-8.8,
+ *   2048^2 11.2-17.9 / 11.6-20.7;
+ *   fp16 NT, 17-64 rows: 1024^2 10.9-11.8 / 8.4-8.6, 2048^2 11.5 / 9.6-10.9,
+ *   512 x 4096 10.9-12.3 / 11.4-12.5; NN, 1-64 rows: 2048^2 11.0-13.9 / 8.8-10.6,
+ *   512 x 4096 11.3 / 11.3.
+ * Up to 16 rows against N x K the decode kernels are level or ahead. */
+static int small_decode(vkblas_dtype_t ab_type, vkblas_op_t op_b, uint32_t M, uint32_t N, uint32_t K) {
+    const uint64_t most = ab_type == VKBLAS_DT_F32 ? 1ull << 20 : 1ull << 22;
+    return g_force_tile < 0 && !g_generic_only && (M >= 17 || op_b == VKBLAS_OP_N) && N >= 32 && K <= 2048 &&
+           (uint64_t)N * K <= most;
+}
+
 /* The body of vkblas_gemm_async.  ws_ext != NULL: the split-K / decode
  * partials go to that buffer of ws_ext_bytes (a call that needs more is
  * rejected with VKBLAS_ERR_PARAM) and nothing is allocated; else the
@@ -746,7 +763,14 @@ static vkblas_status_t gemm_impl(vkblas_dtype_t ab_type, vkblas_dtype_t c_type, 
      * partials: [split][M][N] fp32 for split-K and the split decode kernel,
      * [split][tail_rows][N] for the split tail; with divided K slices
      * (VKB_TILE_64Q) then the parts' sums, VKB_WAVEK_NQ x the partials */
-    int partials = plan.split > 1 && (plan.path == VKBLAS_PATH_SKINNY || plan.path == VKBLAS_PATH_SPLITK ||
+    const int direct = plan.path == VKBLAS_PATH_SKINNY && small_decode(ab_type, op_b, M, N, K);
+    if (direct && plan.split > 1 && !ws_ext) {
+        /* a decode plan with a K split is refused under stream capture
+         * whatever kernel would run it, as ws_acquire refuses it */
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(hs, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return VKBLAS_ERR_INIT;
+    }
+    int partials = !direct && plan.split > 1 && (plan.path == VKBLAS_PATH_SKINNY || plan.path == VKBLAS_PATH_SPLITK ||
                                       plan.path == VKBLAS_PATH_TAIL);
     const size_t part_bytes =
         partials ? (((size_t)plan.split * (plan.path == VKBLAS_PATH_TAIL ? plan.tail_rows : M) * N * sizeof(float) +
@@ -793,7 +817,7 @@ static vkblas_status_t gemm_impl(vkblas_dtype_t ab_type, vkblas_dtype_t c_type, 
     }
 
     float* part = partials ? (float*)((char*)ws + VKB_WS_HEADER) : NULL;
-    if (plan.path == VKBLAS_PATH_SKINNY) {
+    if (plan.path == VKBLAS_PATH_SKINNY && !direct) {
         /* decode; with a K split over workgroups: fp32 partials, fixed-order reduce */
         rc = vkb_launch_skinny(ab, op_b == VKBLAS_OP_T, A, lda, B, ldb, C, ldc, ct, M, N, K, alpha, beta,
                                (int)scalar_mode, alpha_dev, beta_dev, epp, part, partials ? plan.split : 1, stream);
@@ -818,6 +842,7 @@ static vkblas_status_t gemm_impl(vkblas_dtype_t ab_type, vkblas_dtype_t c_type, 
         a.scalar_mode = (int)scalar_mode;
         a.alpha_dev = alpha_dev; a.beta_dev = beta_dev;
         a.generic_only = g_generic_only;
+        a.direct = direct ? 2 : g_force_tile < 0;   /* a forced tile keeps its own kernels */
         a.kernel_out = &kernel;
         a.epi = epp;
         if (plan.path == VKBLAS_PATH_TAIL) {

@@ -4,6 +4,7 @@
 #include "gemm_mfma.hpp"
 #include "gemm_pipe.hpp"
 #include "gemm_wavek.hpp"
+#include "gemm_direct.hpp"
 #include "vkb_launch.h"
 
 namespace vkb {
@@ -60,6 +61,60 @@ static inline uint32_t cu_count() {
 #define VKB_WAVEK_KB16 128
 #endif
 constexpr int WK_KB16 = VKB_WAVEK_KB16;
+
+template <typename T, typename TC, int MF, int NF, int U>
+static int launch_direct_one(const KParams& p, bool ak, bool bk, uint32_t grid, hipStream_t st) {
+    if (ak) {
+        if (bk) hipLaunchKernelGGL((gemm_direct_kernel<T, TC, true, true, MF, NF, U>), dim3(grid), dim3(256), 0, st, p);
+        else hipLaunchKernelGGL((gemm_direct_kernel<T, TC, true, false, MF, NF, U>), dim3(grid), dim3(256), 0, st, p);
+    } else {
+        if (bk) hipLaunchKernelGGL((gemm_direct_kernel<T, TC, false, true, MF, NF, U>), dim3(grid), dim3(256), 0, st, p);
+        else hipLaunchKernelGGL((gemm_direct_kernel<T, TC, false, false, MF, NF, U>), dim3(grid), dim3(256), 0, st, p);
+    }
+    return (int)hipGetLastError();
+}
+
+// gemm_direct_kernel's tile for a call: 64 x 64 where that gives at least 144
+// workgroups, else 32 x 32, and 16 x 32 for fp32 where 32 x 32 gives fewer
+// than 128.  The line is where the larger tile's extra reuse makes up for the
+// CUs it leaves idle (one box, us, 64 / 32 / 16 x 32):
+//   fp32 NT 512 x 1024 x 1024 (128 tiles of 64) 30.9 / 23.2 / 27.0, 768^3 (144)
+//   24.5 / 25.9 / 26.0, 1024^3 31.3 / 42.0 / 49.6; fp32 NN 256^2 x 1024 (64
+//   tiles of 32) 25.1 / 12.0 / 8.2, 384^2 x 2048 (144) TN 37.8 / 16.9 / 20.0;
+//   fp16 NT 512^2 x 1024 11.9 / 8.4, 512 x 1024 x 1024 11.9 / 10.7, 768^3 10.4 / 12.1.
+// Returns 0 if no tile fits the operands (an MN-major operand needs a whole
+// tile in its dimension; a tile's rows must span less than 2^31 bytes).
+template <typename T>
+static uint32_t direct_tile(const vkb_gemm_args* a, uint64_t mats) {
+    auto tiles = [&](uint32_t tm, uint32_t tn) {
+        return (uint64_t)((a->M + tm - 1) / tm) * ((a->N + tn - 1) / tn) * mats;
+    };
+    auto fits = [&](uint32_t tm, uint32_t tn) {
+        // per-lane offsets: the rows of a K-major tile, 32 k rows (or fewer)
+        // of an MN-major one
+        const uint64_t ra = a->a_kmajor ? tm : 32, rb = a->b_kmajor ? tn : 32;
+        return (a->a_kmajor || a->M >= tm) && (a->b_kmajor || a->N >= tn) &&
+               (ra * (uint64_t)a->lda + 64) * sizeof(T) < (1ull << 31) &&
+               (rb * (uint64_t)a->ldb + 64) * sizeof(T) < (1ull << 31);
+    };
+    if (tiles(64, 64) >= 144 && fits(64, 64)) return 64;
+    if ((sizeof(T) == 2 || tiles(32, 32) >= 128) && fits(32, 32)) return 32;
+    if (sizeof(T) == 4 && fits(16, 32)) return 16;
+    return 0;
+}
+
+template <typename T, typename TC>
+static int launch_direct(const vkb_gemm_args* a, KParams p, uint32_t tile, bool ak, bool bk, hipStream_t st) {
+    const uint32_t tm = tile, tn = tile == 16 ? 32 : tile;
+    p.tiles_m = (a->M + tm - 1) / tm;
+    p.tiles_n = (a->N + tn - 1) / tn;
+    const uint64_t grid = (uint64_t)p.tiles_m * p.tiles_n * p.batch * p.split;
+    if (grid == 0 || grid > 0x7fffffffull) return (int)hipErrorInvalidValue;
+    if (tile == 64) return launch_direct_one<T, TC, 4, 4, 4>(p, ak, bk, (uint32_t)grid, st);
+    if (tile == 32) return launch_direct_one<T, TC, 2, 2, 8>(p, ak, bk, (uint32_t)grid, st);
+    if constexpr (sizeof(T) == 4) return launch_direct_one<T, TC, 1, 2, 8>(p, ak, bk, (uint32_t)grid, st);
+    return (int)hipErrorInvalidValue;
+}
 
 template <typename T, typename TC>
 static int launch_gemm_typed(const vkb_gemm_args* a, int tile, hipStream_t st) {
@@ -158,6 +213,43 @@ static int launch_gemm_typed(const vkb_gemm_args* a, int tile, hipStream_t st) {
                               (full || edges_ok);
         const bool pipe_ok = tiles_ok && (p.split == 1 || p.kps % KPAIR == 0) && !a->generic_only &&
                              a->K % KPAIR == 0 && span_a < (1ull << 31) && span_b < (1ull << 31);
+        // Small tiles with fragments straight from memory, where the planner
+        // leaves the choice open (a->direct):
+        //  * instead of the pipelined 128x128 kernel for fp32 on at most 128
+        //    of its tiles, half the CUs (fp32 us, NT / NN / TN: 512 x 1024^2,
+        //    32 tiles, 60 -> 23 / 20 / 18; 1024^3, 64, 60 -> 31 / 27 / 24;
+        //    512 x 4096 x 1024, 128, 61 -> 57 / 49 / 45; 1536^3, 144 tiles,
+        //    89 against 122 / 102 / 85).  16-bit inputs stay there: level at
+        //    32 tiles, ahead from 36 on (768 x 1024 x 3072 fp16 22 against 26);
+        //  * instead of the generic kernel with edge handling, but for many
+        //    tiles with a short K, where the four waves have too little to
+        //    share (96 x 197 x 197 x 64 fp16 9.8 against 15.0), and for many
+        //    tiles of aligned 16-bit operands, which that kernel loads as
+        //    vectors (fp16 NT, 64 x 64 tiles: 128 x 32003 x 1024, 1002 of them,
+        //    26 against 48; 1000^3, 256, 22 against 12; unaligned 999 x 1001 x
+        //    1003 NT / TN 113 / 186 against 21 / 12);
+        //  * instead of the generic kernel on whole tiles where 64 x 64 ones
+        //    would leave CUs idle (fp32 NT 512^2 x 2048 49 -> 25; 64 x 1024 x 64 x
+        //    1024 bf16, 1024 tiles: 32 against 50); split-K pass 1 on whole tiles
+        //    is the wave-K kernel's.
+        if (a->direct && !p.ptr_array && !a->generic_only &&
+            (tile == VKB_TILE_64 || tile == VKB_TILE_128 || tile == VKB_TILE_256)) {
+            const uint64_t mats = (uint64_t)p.batch * p.split;
+            const uint64_t t64 = (uint64_t)((a->M + 63) / 64) * ((a->N + 63) / 64) * mats;
+            const bool pipe = pipe_ok && tile != VKB_TILE_64;
+            const uint32_t klen = p.split > 1 ? p.kps : a->K;
+            const bool want = a->direct == 2 ? true
+                            : pipe ? sizeof(T) == 4 && tile == VKB_TILE_128 && p.split == 1 && grid <= 128
+                            : full ? p.split == 1 && t64 < 192
+                            : t64 <= 512 ? true
+                                   : (uint64_t)klen * sizeof(T) >= 512 && (sizeof(T) == 4 || !p.vec_a || !p.vec_b);
+            const uint32_t dt = want ? direct_tile<T>(a, mats) : 0;
+            if (dt) {
+                // a decode plan's call still reports a decode kernel
+                report(a->direct == 2 ? VKB_KERN_SKINNY : VKB_KERN_DIRECT);
+                return launch_direct<T, TC>(a, p, dt, ak, bk, st);
+            }
+        }
         if (tile == VKB_TILE_256 && pipe_ok) {
             report(VKB_KERN_PIPE256);
             if (ak) {

@@ -33,8 +33,10 @@ enum {
     VKB_KERN_PIPE128 = 4,          /* gemm_pipe_kernel, 128x128, 2 stages   */
     VKB_KERN_PIPE128_4 = 5,        /* gemm_pipe_kernel, 128x128, 4 stages   */
     VKB_KERN_SKINNY = 6,           /* decode kernels (skinny.hip)           */
-    VKB_KERN_WAVEK = 7             /* gemm_wavek_kernel: split-K pass 1 on
+    VKB_KERN_WAVEK = 7,            /* gemm_wavek_kernel: split-K pass 1 on
                                       32x32 / 64x64 tiles, K over the waves */
+    VKB_KERN_DIRECT = 8            /* gemm_direct_kernel: small tiles, K over
+                                      the waves, no LDS in the K loop       */
 };
 
 /* GEMM tile configurations (block tile BM x BN, 4 waves, BK = 128 bytes) */
@@ -113,6 +115,9 @@ typedef struct vkb_gemm_args {
      * last to arrive writes the slice's partial to C. */
     float* qpart;
     uint32_t* qcnt;
+    /* 1: gemm_direct_kernel instead of the tile's kernel where the launcher's
+     * rule finds it faster; 2: wherever it can run; 0: never */
+    int direct;
 } vkb_gemm_args;
 
 /* Tile-config properties the dispatcher plans with. */
