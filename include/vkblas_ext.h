@@ -56,8 +56,10 @@ typedef enum {
     VKBLAS_KERNEL_SKINNY = 6,           /* decode plans (vkblas_last_path skinny)  */
     VKBLAS_KERNEL_WAVEK = 7,            /* split-K pass 1 on 32 x 32 / 64 x 64
                                            tiles, the slice's K over the waves  */
-    VKBLAS_KERNEL_DIRECT = 8            /* small tiles, K over the waves, MFMA
+    VKBLAS_KERNEL_DIRECT = 8,           /* small tiles, K over the waves, MFMA
                                            fragments straight from memory       */
+    VKBLAS_KERNEL_FLOW = 9              /* 16-bit 128 x 128 / 128 x 64 tiles, any
+                                           M, N and C, K in 16-byte chunks      */
 } vkblas_kernel_t;
 
 typedef struct {

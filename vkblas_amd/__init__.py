@@ -132,7 +132,7 @@ def last_path() -> int:
 
 # vkblas_kernel_t (include/vkblas_ext.h)
 KERNEL_NONE, KERNEL_GENERIC, KERNEL_GENERIC_CHECKED, KERNEL_PIPE256, KERNEL_PIPE128, KERNEL_PIPE128_4, \
-    KERNEL_SKINNY, KERNEL_WAVEK, KERNEL_DIRECT = range(9)
+    KERNEL_SKINNY, KERNEL_WAVEK, KERNEL_DIRECT, KERNEL_FLOW = range(10)
 
 
 def workspace_release() -> None:

@@ -5,6 +5,7 @@
 #include "gemm_pipe.hpp"
 #include "gemm_wavek.hpp"
 #include "gemm_direct.hpp"
+#include "gemm_flow.hpp"
 #include "vkb_launch.h"
 
 namespace vkb {
@@ -72,6 +73,61 @@ static int launch_direct_one(const KParams& p, bool ak, bool bk, uint32_t grid, 
         else hipLaunchKernelGGL((gemm_direct_kernel<T, TC, false, false, MF, NF, U>), dim3(grid), dim3(256), 0, st, p);
     }
     return (int)hipGetLastError();
+}
+
+template <typename T, typename TC, int BN, int NST, int WAVES>
+static int launch_flow_one(const KParams& p, bool ak, bool bk, uint32_t grid, hipStream_t st) {
+    const dim3 wg(64 * WAVES);
+    if (ak) {
+        if (bk) hipLaunchKernelGGL((gemm_flow_kernel<T, TC, true, true, BN, NST, WAVES>), dim3(grid), wg, 0, st, p);
+        else hipLaunchKernelGGL((gemm_flow_kernel<T, TC, true, false, BN, NST, WAVES>), dim3(grid), wg, 0, st, p);
+    } else {
+        if (bk) hipLaunchKernelGGL((gemm_flow_kernel<T, TC, false, true, BN, NST, WAVES>), dim3(grid), wg, 0, st, p);
+        else hipLaunchKernelGGL((gemm_flow_kernel<T, TC, false, false, BN, NST, WAVES>), dim3(grid), wg, 0, st, p);
+    }
+    return (int)hipGetLastError();
+}
+
+// Whether gemm_flow_kernel takes a call: 16-byte aligned 16-bit operands and
+// leading dimensions (vec_a, vec_b), K in whole 16-byte chunks where an operand
+// is K-major, the row dimension of an MN-major one a multiple of 8, every
+// offset below 2 GiB.
+template <typename T>
+static bool flow_ok(const vkb_gemm_args* a, const KParams& p) {
+    if (sizeof(T) != 2 || p.ptr_array || !p.vec_a || !p.vec_b) return false;
+    const uint64_t span_a = ((uint64_t)(a->a_kmajor ? 128 : a->K + 64) * (uint64_t)a->lda + (a->a_kmajor ? a->K + 64 : a->M)) * 2;
+    const uint64_t span_b = ((uint64_t)(a->b_kmajor ? 128 : a->K + 64) * (uint64_t)a->ldb + (a->b_kmajor ? a->K + 64 : a->N)) * 2;
+    return (a->a_kmajor ? a->K % 8 == 0 : a->M % 8 == 0) && (a->b_kmajor ? a->K % 8 == 0 : a->N % 8 == 0) &&
+           span_a < (1ull << 31) && span_b < (1ull << 31);
+}
+
+// gemm_flow_kernel's form, from the number of 128 x 128 tiles t (one box, fp16 us):
+//  * N of one 64-column tile, or t at most half the CUs: 128 x 64 tiles, three
+//    stages, two workgroups per CU (1000^3, t = 64, 11.2 against 13.8 on 128 x 128;
+//    1280 x 1280 x 1000, 100, 11.2 / 13.7; 1536 x 1536 x 1000, 144, 15.9 / 13.5);
+//  * up to one per CU: 128 x 128, three stages, eight waves (96 KB, one workgroup
+//    per CU: two waves per SIMD; 2001 x 2000 x 2000 23.6 against 30.3 with two
+//    stages and two workgroups of four waves per CU, 25.9 with four waves);
+//  * more: 128 x 128, two stages, two workgroups per CU (4000^3 145 against 166);
+//    K of a single step: one stage and three or four workgroups per CU (64 x 1024 x
+//    1024 x 64 29.7 against 34.7 with two stages).
+template <typename T, typename TC>
+static int launch_flow(const vkb_gemm_args* a, KParams p, bool ak, bool bk, hipStream_t st) {
+    if constexpr (sizeof(T) == 2) {
+        const uint64_t mats = (uint64_t)p.batch * p.split;
+        p.tiles_m = (a->M + 127) / 128;
+        p.tiles_n = (a->N + 127) / 128;
+        const uint64_t t = (uint64_t)p.tiles_m * p.tiles_n * mats;
+        const bool narrow = a->N <= 64 || t <= 128;
+        if (narrow) p.tiles_n = (a->N + 63) / 64;
+        const uint64_t grid = (uint64_t)p.tiles_m * p.tiles_n * mats;
+        if (grid == 0 || grid > 0x7fffffffull) return (int)hipErrorInvalidValue;
+        if (narrow) return launch_flow_one<T, TC, 64, 3, 4>(p, ak, bk, (uint32_t)grid, st);
+        if (t <= 256) return launch_flow_one<T, TC, 128, 3, 8>(p, ak, bk, (uint32_t)grid, st);
+        if ((p.split > 1 ? p.kps : a->K) <= 64) return launch_flow_one<T, TC, 128, 1, 4>(p, ak, bk, (uint32_t)grid, st);
+        return launch_flow_one<T, TC, 128, 2, 4>(p, ak, bk, (uint32_t)grid, st);
+    }
+    return (int)hipErrorInvalidValue;
 }
 
 // gemm_direct_kernel's tile for a call: 64 x 64 where that gives at least 144
@@ -213,34 +269,43 @@ static int launch_gemm_typed(const vkb_gemm_args* a, int tile, hipStream_t st) {
                               (full || edges_ok);
         const bool pipe_ok = tiles_ok && (p.split == 1 || p.kps % KPAIR == 0) && !a->generic_only &&
                              a->K % KPAIR == 0 && span_a < (1ull << 31) && span_b < (1ull << 31);
-        // Small tiles with fragments straight from memory, where the planner
-        // leaves the choice open (a->direct):
-        //  * instead of the pipelined 128x128 kernel for fp32 on at most 128
-        //    of its tiles, half the CUs (fp32 us, NT / NN / TN: 512 x 1024^2,
-        //    32 tiles, 60 -> 23 / 20 / 18; 1024^3, 64, 60 -> 31 / 27 / 24;
-        //    512 x 4096 x 1024, 128, 61 -> 57 / 49 / 45; 1536^3, 144 tiles,
-        //    89 against 122 / 102 / 85).  16-bit inputs stay there: level at
-        //    32 tiles, ahead from 36 on (768 x 1024 x 3072 fp16 22 against 26);
-        //  * instead of the generic kernel with edge handling, but for many
-        //    tiles with a short K, where the four waves have too little to
-        //    share (96 x 197 x 197 x 64 fp16 9.8 against 15.0), and for many
-        //    tiles of aligned 16-bit operands, which that kernel loads as
-        //    vectors (fp16 NT, 64 x 64 tiles: 128 x 32003 x 1024, 1002 of them,
-        //    26 against 48; 1000^3, 256, 22 against 12; unaligned 999 x 1001 x
-        //    1003 NT / TN 113 / 186 against 21 / 12);
-        //  * instead of the generic kernel on whole tiles where 64 x 64 ones
-        //    would leave CUs idle (fp32 NT 512^2 x 2048 49 -> 25; 64 x 1024 x 64 x
-        //    1024 bf16, 1024 tiles: 32 against 50); split-K pass 1 on whole tiles
-        //    is the wave-K kernel's.
+        // Where the planner leaves the choice open (a->direct) and the wave-K
+        // kernel does not take the call (split-K pass 1 on whole 64x64 tiles):
+        //  * aligned 16-bit operands that the pipelined kernel does not take:
+        //    gemm_flow_kernel from 144 tiles of 64x64 on (fp16 NT 2000 x 2001 x 1000
+        //    26 -> 19 us, TN 2000^3 136 -> 24, 64 x 512 x 512 x 80 35 -> 12, 64 x 1024 x
+        //    1024 x 64 58 -> 30 against the generic kernel; 768 x 768 x 1000, 144
+        //    tiles, 11.9 -> 10.9 against the direct one, 640 x 640, 100, 10.4 / 10.9);
+        //  * gemm_direct_kernel (small tiles, fragments straight from memory)
+        //    - instead of the pipelined 128x128 kernel for fp32 on at most 128
+        //      of its tiles, half the CUs (fp32 us, NT / NN / TN: 512 x 1024^2,
+        //      32 tiles, 60 -> 23 / 20 / 18; 1024^3, 64, 60 -> 31 / 27 / 24;
+        //      512 x 4096 x 1024, 128, 61 -> 57 / 49 / 45; 1536^3, 144 tiles,
+        //      89 against 122 / 102 / 85).  16-bit inputs stay there: level at
+        //      32 tiles, ahead from 36 on (768 x 1024 x 3072 fp16 22 against 26);
+        //    - instead of the generic kernel with edge handling, but for many
+        //      tiles with a short K, where the four waves have too little to
+        //      share (96 x 197 x 197 x 64 fp16 9.8 against 15.0), and for many
+        //      tiles of aligned 16-bit operands, which that kernel loads as
+        //      vectors (fp16 NT, 64 x 64 tiles: 128 x 32003 x 1024, 1002 of them,
+        //      26 against 48; unaligned 999 x 1001 x 1003 NT / TN 113 / 186
+        //      against 21 / 12);
+        //    - instead of the generic kernel on whole tiles where 64 x 64 ones
+        //      would leave CUs idle (fp32 NT 512^2 x 2048 49 -> 25).
         if (a->direct && !p.ptr_array && !a->generic_only &&
-            (tile == VKB_TILE_64 || tile == VKB_TILE_128 || tile == VKB_TILE_256)) {
+            (tile == VKB_TILE_64 || tile == VKB_TILE_128 || tile == VKB_TILE_256) &&
+            !(tile == VKB_TILE_64 && p.split > 1 && full)) {
             const uint64_t mats = (uint64_t)p.batch * p.split;
             const uint64_t t64 = (uint64_t)((a->M + 63) / 64) * ((a->N + 63) / 64) * mats;
             const bool pipe = pipe_ok && tile != VKB_TILE_64;
+            if (a->direct == 1 && !pipe && t64 >= 144 && flow_ok<T>(a, p)) {
+                report(VKB_KERN_FLOW);
+                return launch_flow<T, TC>(a, p, ak, bk, st);
+            }
             const uint32_t klen = p.split > 1 ? p.kps : a->K;
             const bool want = a->direct == 2 ? true
                             : pipe ? sizeof(T) == 4 && tile == VKB_TILE_128 && p.split == 1 && grid <= 128
-                            : full ? p.split == 1 && t64 < 192
+                            : full ? t64 < 192
                             : t64 <= 512 ? true
                                    : (uint64_t)klen * sizeof(T) >= 512 && (sizeof(T) == 4 || !p.vec_a || !p.vec_b);
             const uint32_t dt = want ? direct_tile<T>(a, mats) : 0;

@@ -35,8 +35,10 @@ enum {
     VKB_KERN_SKINNY = 6,           /* decode kernels (skinny.hip)           */
     VKB_KERN_WAVEK = 7,            /* gemm_wavek_kernel: split-K pass 1 on
                                       32x32 / 64x64 tiles, K over the waves */
-    VKB_KERN_DIRECT = 8            /* gemm_direct_kernel: small tiles, K over
+    VKB_KERN_DIRECT = 8,           /* gemm_direct_kernel: small tiles, K over
                                       the waves, no LDS in the K loop       */
+    VKB_KERN_FLOW = 9              /* gemm_flow_kernel: 16-bit 128x128 and
+                                      128x64 tiles, any K % 8, M, N and C   */
 };
 
 /* GEMM tile configurations (block tile BM x BN, 4 waves, BK = 128 bytes) */
@@ -115,8 +117,9 @@ typedef struct vkb_gemm_args {
      * last to arrive writes the slice's partial to C. */
     float* qpart;
     uint32_t* qcnt;
-    /* 1: gemm_direct_kernel instead of the tile's kernel where the launcher's
-     * rule finds it faster; 2: wherever it can run; 0: never */
+    /* 1: gemm_flow_kernel or gemm_direct_kernel instead of the tile's kernel
+     * where the launcher's rule finds them faster; 2: gemm_direct_kernel
+     * wherever it can run; 0: neither */
     int direct;
 } vkb_gemm_args;
 
