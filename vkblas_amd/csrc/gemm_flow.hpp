@@ -43,7 +43,10 @@ namespace vkb {
 constexpr int flow_wg_per_cu(int BN, int NST, bool kmajor) {
     return NST == 1 ? (kmajor ? 4 : 3) : NST * (128 + BN) * 128 > 80 * 1024 ? 1 : 2;
 }
-template <typename T, typename TC, bool AK, bool BKM, int BN, int NST, int WAVES>
+// EARLY: beta's matrix is read before the K loop, which then hides its latency
+// (bf16 -> fp32 TN 4096 x 1024 x 512, beta = 1: 14.5 -> 11.0 us); a form of its own,
+// as its registers and the early scalars cost the others 3 % (attention bf16).
+template <typename T, typename TC, bool AK, bool BKM, int BN, int NST, int WAVES, bool EARLY = false>
 __global__ __launch_bounds__(64 * WAVES, flow_wg_per_cu(BN, NST, AK && BKM) * WAVES / 4)
 void gemm_flow_kernel(KParams p) {
     static_assert(sizeof(T) == 2, "16-bit operands");
@@ -202,6 +205,27 @@ void gemm_flow_kernel(KParams p) {
         }
     };
 
+    // the epilogue's share of C: row segments of WN columns, CV of them per lane
+    constexpr int CV = 16 / (int)sizeof(TC);
+    constexpr int LPR = WN / CV;                      // lanes per row
+    constexpr int IT = 16 * LPR / 64;                 // rounds per 16 rows
+    typedef TC cvec __attribute__((ext_vector_type(CV)));
+    typedef cvec cvec_any __attribute__((aligned(2), may_alias));
+    float alpha, beta;
+    cvec old[EARLY ? NFM : 1][EARLY ? IT : 1];
+    if constexpr (EARLY) {
+        load_scalars(p, alpha, beta);
+        const int n = n0 + wn * WN + lane % LPR * CV;
+        const TC* Ci = (const TC*)p.epi.cin + (int64_t)b * p.epi.scin;
+#pragma unroll
+        for (int i = 0; i < NFM; ++i)
+#pragma unroll
+            for (int it = 0; it < IT; ++it) {
+                const int m = m0 + wm * WM + 16 * i + it * (64 / LPR) + lane / LPR;
+                if (m < M && n + CV <= N) old[i][it] = *(const cvec_any*)(Ci + (int64_t)m * p.epi.ldcin + n);
+            }
+    }
+
     floatx4 acc[NFM][NFN];
 #pragma unroll
     for (int i = 0; i < NFM; ++i)
@@ -250,15 +274,10 @@ void gemm_flow_kernel(KParams p) {
 
     // ---- epilogue ----
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // the stages are free
-    float alpha, beta;
-    load_scalars(p, alpha, beta);
+    if constexpr (!EARLY) load_scalars(p, alpha, beta);
     float* rows = (float*)lds + wave * 16 * EROW;
-    constexpr int CV = 16 / (int)sizeof(TC);          // columns per lane
-    constexpr int LPR = WN / CV;                      // lanes per row
     TC* Cb = (TC*)p.C + (int64_t)b * p.sc + (int64_t)s * p.s_split;
     const TC* Ci = (const TC*)p.epi.cin + (int64_t)b * p.epi.scin;
-    typedef TC cvec __attribute__((ext_vector_type(CV)));
-    typedef cvec cvec_any __attribute__((aligned(2), may_alias));
     const int c = lane % LPR * CV;                    // this lane's first column of the wave's
     const int n = n0 + wn * WN + c;
     float bias[CV];
@@ -272,7 +291,7 @@ void gemm_flow_kernel(KParams p) {
         // compiler from reordering the cross-lane read-back
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
-        for (int it = 0; it < 16 * LPR / 64; ++it) {
+        for (int it = 0; it < IT; ++it) {
             const int r = it * (64 / LPR) + lane / LPR;
             const int m = m0 + wm * WM + 16 * i + r;
             float x[CV];
@@ -287,7 +306,9 @@ void gemm_flow_kernel(KParams p) {
                 const TC* cin = Ci + (int64_t)m * p.epi.ldcin + n;
                 if (n + CV <= N) {
                     if (beta != 0.0f) {
-                        const cvec o = *(const cvec_any*)cin;
+                        cvec o;
+                        if constexpr (EARLY) o = old[i][it];
+                        else o = *(const cvec_any*)cin;
 #pragma unroll
                         for (int e = 0; e < CV; ++e) x[e] += beta * (float)o[e];
                     }

@@ -75,15 +75,15 @@ static int launch_direct_one(const KParams& p, bool ak, bool bk, uint32_t grid, 
     return (int)hipGetLastError();
 }
 
-template <typename T, typename TC, int BN, int NST, int WAVES>
+template <typename T, typename TC, int BN, int NST, int WAVES, bool EARLY = false>
 static int launch_flow_one(const KParams& p, bool ak, bool bk, uint32_t grid, hipStream_t st) {
     const dim3 wg(64 * WAVES);
     if (ak) {
-        if (bk) hipLaunchKernelGGL((gemm_flow_kernel<T, TC, true, true, BN, NST, WAVES>), dim3(grid), wg, 0, st, p);
-        else hipLaunchKernelGGL((gemm_flow_kernel<T, TC, true, false, BN, NST, WAVES>), dim3(grid), wg, 0, st, p);
+        if (bk) hipLaunchKernelGGL((gemm_flow_kernel<T, TC, true, true, BN, NST, WAVES, EARLY>), dim3(grid), wg, 0, st, p);
+        else hipLaunchKernelGGL((gemm_flow_kernel<T, TC, true, false, BN, NST, WAVES, EARLY>), dim3(grid), wg, 0, st, p);
     } else {
-        if (bk) hipLaunchKernelGGL((gemm_flow_kernel<T, TC, false, true, BN, NST, WAVES>), dim3(grid), wg, 0, st, p);
-        else hipLaunchKernelGGL((gemm_flow_kernel<T, TC, false, false, BN, NST, WAVES>), dim3(grid), wg, 0, st, p);
+        if (bk) hipLaunchKernelGGL((gemm_flow_kernel<T, TC, false, true, BN, NST, WAVES, EARLY>), dim3(grid), wg, 0, st, p);
+        else hipLaunchKernelGGL((gemm_flow_kernel<T, TC, false, false, BN, NST, WAVES, EARLY>), dim3(grid), wg, 0, st, p);
     }
     return (int)hipGetLastError();
 }
@@ -122,7 +122,10 @@ static int launch_flow(const vkb_gemm_args* a, KParams p, bool ak, bool bk, hipS
         if (narrow) p.tiles_n = (a->N + 63) / 64;
         const uint64_t grid = (uint64_t)p.tiles_m * p.tiles_n * mats;
         if (grid == 0 || grid > 0x7fffffffull) return (int)hipErrorInvalidValue;
+        const bool early = a->scalar_mode == VKB_SCALAR_HOST && a->beta != 0.0f;   // beta's matrix before the K loop
+        if (narrow && early) return launch_flow_one<T, TC, 64, 3, 4, true>(p, ak, bk, (uint32_t)grid, st);
         if (narrow) return launch_flow_one<T, TC, 64, 3, 4>(p, ak, bk, (uint32_t)grid, st);
+        if (t <= 256 && early) return launch_flow_one<T, TC, 128, 3, 8, true>(p, ak, bk, (uint32_t)grid, st);
         if (t <= 256) return launch_flow_one<T, TC, 128, 3, 8>(p, ak, bk, (uint32_t)grid, st);
         if ((p.split > 1 ? p.kps : a->K) <= 64) return launch_flow_one<T, TC, 128, 1, 4>(p, ak, bk, (uint32_t)grid, st);
         return launch_flow_one<T, TC, 128, 2, 4>(p, ak, bk, (uint32_t)grid, st);
@@ -276,6 +279,10 @@ static int launch_gemm_typed(const vkb_gemm_args* a, int tile, hipStream_t st) {
         //    26 -> 19 us, TN 2000^3 136 -> 24, 64 x 512 x 512 x 80 35 -> 12, 64 x 1024 x
         //    1024 x 64 58 -> 30 against the generic kernel; 768 x 768 x 1000, 144
         //    tiles, 11.9 -> 10.9 against the direct one, 640 x 640, 100, 10.4 / 10.9);
+        //    and instead of the pipelined 128x128 kernel on one wave of tiles
+        //    where beta adds to C after at most 1024 k, as it reads C before the K
+        //    loop and not after it (bf16 -> fp32 TN, 4096 x 1024 x 512 13.2 -> 11.0 us,
+        //    1024 x 1024 x 512 10.9 -> 8.4, K = 1024 18.5 -> 17.8, but 2048 24.9 -> 26.2);
         //  * gemm_direct_kernel (small tiles, fragments straight from memory)
         //    - instead of the pipelined 128x128 kernel for fp32 on at most 128
         //      of its tiles, half the CUs (fp32 us, NT / NN / TN: 512 x 1024^2,
@@ -298,7 +305,9 @@ static int launch_gemm_typed(const vkb_gemm_args* a, int tile, hipStream_t st) {
             const uint64_t mats = (uint64_t)p.batch * p.split;
             const uint64_t t64 = (uint64_t)((a->M + 63) / 64) * ((a->N + 63) / 64) * mats;
             const bool pipe = pipe_ok && tile != VKB_TILE_64;
-            if (a->direct == 1 && !pipe && t64 >= 144 && flow_ok<T>(a, p)) {
+            const bool add = pipe && tile == VKB_TILE_128 && p.split == 1 && grid <= 256 &&
+                             a->scalar_mode == VKB_SCALAR_HOST && a->beta != 0.0f && a->K <= 1024;
+            if (a->direct == 1 && ((!pipe && t64 >= 144) || add) && flow_ok<T>(a, p)) {
                 report(VKB_KERN_FLOW);
                 return launch_flow<T, TC>(a, p, ak, bk, st);
             }
