@@ -10,6 +10,8 @@ and ``__graft_entry__``: it loads the built library with ctypes and mirrors the
 engine entry points (``vkblas_gemm_f32`` / ``vkblas_gemm_f16`` of the
 reference's ``src/vkblas.h:27-77``) with the same argument meaning and status
 codes.  There is no fallback: if the library is missing, loading raises.
+The asynchronous GEMMs go through ``_call`` (csrc/pycall.c), which converts
+their arguments natively; arguments it does not know go through ctypes.
 """
 from __future__ import annotations
 
@@ -23,6 +25,8 @@ LIB_NAME = "libvkblas_hipblas.so"
 LIB_PATH = os.path.join(HERE, LIB_NAME)
 # the host dispatcher and kernels, opened by LIB_PATH's first call
 ENGINE_PATH = os.path.join(HERE, "libvkblas_engine.so")
+# the binding's calls (module vkblas_amd._call)
+CALL_PATH = os.path.join(HERE, "_call.so")
 
 # vkblas_status_t (reference src/vkblas.h:6-12)
 OK, ERR_INIT, ERR_IMPORT, ERR_PARAM, ERR_FALLBACK = 0, 1, 2, 3, 4
@@ -57,6 +61,8 @@ class Plan(ctypes.Structure):
 
 
 _lib = None
+_native = None      # vkblas_amd._call.gemm_ex, set by load()
+_ex_addr = 0        # address of vkblas_gemm_ex_async
 
 _u32, _i64, _f, _vp, _int = ctypes.c_uint32, ctypes.c_int64, ctypes.c_float, ctypes.c_void_p, ctypes.c_int
 _ENGINE_ARGS = [_int, _int, _u32, _u32, _u32, _f, _vp, _u32, _vp, _u32, _f, _vp, _u32, _u32, _i64, _i64, _i64]
@@ -69,10 +75,10 @@ def build(jobs: int = 8) -> None:
 
 def load():
     """Load the built library (raises if it has not been built)."""
-    global _lib
+    global _lib, _native, _ex_addr
     if _lib is not None:
         return _lib
-    for path in (LIB_PATH, ENGINE_PATH):
+    for path in (LIB_PATH, ENGINE_PATH, CALL_PATH):
         if not os.path.exists(path):
             raise RuntimeError(f"{path} is missing: run __graft_entry__.build() (make -C vkblas_amd)")
     L = ctypes.CDLL(LIB_PATH)
@@ -102,6 +108,8 @@ def load():
     L.vkblas_gemm_noalloc_async.argtypes = L.vkblas_gemm_async.argtypes
     L.vkblas_gemm_noalloc_async.restype = _int
     L.vkblas_noalloc_scratch_bytes.restype = ctypes.c_size_t
+    from . import _call
+    _native, _ex_addr = _call.gemm_ex, ctypes.cast(L.vkblas_gemm_ex_async, ctypes.c_void_p).value
     _lib = L
     return L
 
@@ -152,9 +160,15 @@ def gemm_async(ab_type, c_type, op_a, op_b, M, N, K, alpha, A, lda, B, ldb, beta
                split_k=0, stream=None, check=True) -> int:
     """vkblas_gemm_async on raw device pointers (ints).  Row-major engine
     contract of src/vkblas.h:21-26.  Returns the status (raises if check)."""
-    st = load().vkblas_gemm_async(ab_type, c_type, op_a, op_b, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc,
-                                  batch, stride_a, stride_b, stride_c, scalar_mode, alpha_dev, beta_dev, split_k,
-                                  stream)
+    if _lib is None:
+        load()
+    st = _native(_ex_addr, ab_type, c_type, op_a, op_b, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, batch,
+                 stride_a, stride_b, stride_c, scalar_mode, alpha_dev, beta_dev, split_k, 0, None, 0, 0, None, 0,
+                 stream)
+    if st is None:
+        st = _lib.vkblas_gemm_async(ab_type, c_type, op_a, op_b, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc,
+                                    batch, stride_a, stride_b, stride_c, scalar_mode, alpha_dev, beta_dev, split_k,
+                                    stream)
     if check and st != OK:
         raise VkblasError(st, "vkblas_gemm_async")
     return st
@@ -166,10 +180,16 @@ def gemm_ex_async(ab_type, c_type, op_a, op_b, M, N, K, alpha, A, lda, B, ldb, b
                   check=True) -> int:
     """vkblas_gemm_ex_async: gemm_async with a separate C input (c_in, beta's
     matrix) and a bias vector (one value per column n of C)."""
-    ep = Epilogue(c_in, ldc_in, stride_c_in, bias, bias_type)
-    st = load().vkblas_gemm_ex_async(ab_type, c_type, op_a, op_b, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc,
-                                     batch, stride_a, stride_b, stride_c, scalar_mode, alpha_dev, beta_dev, split_k,
-                                     ctypes.byref(ep), stream)
+    if _lib is None:
+        load()
+    st = _native(_ex_addr, ab_type, c_type, op_a, op_b, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, batch,
+                 stride_a, stride_b, stride_c, scalar_mode, alpha_dev, beta_dev, split_k, 1, c_in, ldc_in,
+                 stride_c_in, bias, bias_type, stream)
+    if st is None:
+        ep = Epilogue(c_in, ldc_in, stride_c_in, bias, bias_type)
+        st = _lib.vkblas_gemm_ex_async(ab_type, c_type, op_a, op_b, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc,
+                                       batch, stride_a, stride_b, stride_c, scalar_mode, alpha_dev, beta_dev,
+                                       split_k, ctypes.byref(ep), stream)
     if check and st != OK:
         raise VkblasError(st, "vkblas_gemm_ex_async")
     return st
