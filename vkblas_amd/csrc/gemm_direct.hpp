@@ -36,7 +36,6 @@ typedef uint32_t u32x2_d __attribute__((ext_vector_type(2)));
 // gfx950's vector loads take it, the compiler splits nothing)
 typedef uint32_t u32_any __attribute__((aligned(2), may_alias));
 typedef u32x2_d u32x2_any __attribute__((aligned(2), may_alias));
-typedef u32x4 u32x4_any __attribute__((aligned(2), may_alias));
 template <int N>
 __device__ __forceinline__ void ld_dwords(uint32_t* d, const void* p) {
     static_assert(N == 1 || N == 2 || N == 4, "1, 2 or 4 dwords");

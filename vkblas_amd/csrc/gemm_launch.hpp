@@ -162,6 +162,25 @@ static uint32_t direct_tile(const vkb_gemm_args* a, uint64_t mats) {
     return 0;
 }
 
+// The generic kernel's 128 x 128 tiles, each operand read once, against many
+// small tiles whose operands come from the caches over and over: the line by
+// layout, since an operand read along K costs gemm_direct_kernel more loads and
+// one read across it costs the generic kernel a transpose (unaligned, us,
+// generic / direct, in brackets the tiles of 64 x 64):
+//   fp32 NT 999^3 (256) 81 / 32, 1500^2 x 1003 (576) 82 / 83, 2001 x 2003 x 2005
+//   (1024) 156 / 214; NN 228 / 197, TN 276 / 161 there, 321 / 282 and 358 / 237 at
+//   4001 x 3001 x 1003 (2961): direct throughout;
+//   fp16 NT 333 x 1001 x 2003 (96) 27 / 42, 999^3 25 / 22, 777 x 3001 x 1003 (611)
+//   26 / 58, 2001^3 46 / 169; NN 333 x 1001 x 2003 46 / 27, 100 x 10007 x 777 (314)
+//   30 / 27, 1500^2 35 / 44, 2001^3 62 / 117; TN 2001^3 81 / 71, 4001 x 3001 x
+//   1003 88 / 135.
+template <typename T>
+static bool direct_loses(bool ak, bool bk, uint64_t t64, uint32_t klen) {
+    if (sizeof(T) == 4) return ak && bk && t64 >= 560;
+    if (ak && bk) return t64 > 256 || (t64 >= 96 && klen >= 1536);
+    return t64 >= (ak || bk ? 400 : 1536);
+}
+
 template <typename T, typename TC>
 static int launch_direct(const vkb_gemm_args* a, KParams p, uint32_t tile, bool ak, bool bk, hipStream_t st) {
     const uint32_t tm = tile, tn = tile == 16 ? 32 : tile;
@@ -290,13 +309,10 @@ static int launch_gemm_typed(const vkb_gemm_args* a, int tile, hipStream_t st) {
         //      512 x 4096 x 1024, 128, 61 -> 57 / 49 / 45; 1536^3, 144 tiles,
         //      89 against 122 / 102 / 85).  16-bit inputs stay there: level at
         //      32 tiles, ahead from 36 on (768 x 1024 x 3072 fp16 22 against 26);
-        //    - instead of the generic kernel with edge handling, but for many
-        //      tiles with a short K, where the four waves have too little to
-        //      share (96 x 197 x 197 x 64 fp16 9.8 against 15.0), and for many
-        //      tiles of aligned 16-bit operands, which that kernel loads as
-        //      vectors (fp16 NT, 64 x 64 tiles: 128 x 32003 x 1024, 1002 of them,
-        //      26 against 48; unaligned 999 x 1001 x 1003 NT / TN 113 / 186
-        //      against 21 / 12);
+        //    - instead of the generic kernel with edge handling, but not where
+        //      direct_loses (many tiles) or for many tiles with a short K, where
+        //      the four waves have too little to share (96 x 197 x 197 x 64 fp16
+        //      9.8 against 15.0);
         //    - instead of the generic kernel on whole tiles where 64 x 64 ones
         //      would leave CUs idle (fp32 NT 512^2 x 2048 49 -> 25).
         if (a->direct && !p.ptr_array && !a->generic_only &&
@@ -315,8 +331,8 @@ static int launch_gemm_typed(const vkb_gemm_args* a, int tile, hipStream_t st) {
             const bool want = a->direct == 2 ? true
                             : pipe ? sizeof(T) == 4 && tile == VKB_TILE_128 && p.split == 1 && grid <= 128
                             : full ? t64 < 192
-                            : t64 <= 512 ? true
-                                   : (uint64_t)klen * sizeof(T) >= 512 && (sizeof(T) == 4 || !p.vec_a || !p.vec_b);
+                                   : !direct_loses<T>(ak, bk, t64, klen) &&
+                                         ((uint64_t)klen * sizeof(T) >= 512 || t64 <= 512);
             const uint32_t dt = want ? direct_tile<T>(a, mats) : 0;
             if (dt) {
                 // a decode plan's call still reports a decode kernel

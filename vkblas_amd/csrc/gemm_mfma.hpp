@@ -119,32 +119,42 @@ __device__ __forceinline__ void load_scalars(const KParams& p, float& alpha, flo
     }
 }
 
-// one element as raw bits, zero when out of range
+// 16 bytes from an address of any element alignment (2 bytes: gfx950's vector
+// loads take it)
+typedef u32x4 u32x4_any __attribute__((aligned(2), may_alias));
 template <typename T>
-__device__ __forceinline__ uint32_t ld_bits(const T* p, bool ok) {
-    if constexpr (sizeof(T) == 4) {
-        return ok ? *(const uint32_t*)p : 0u;
-    } else {
-        return ok ? (uint32_t)(*(const uint16_t*)p) : 0u;
-    }
+__device__ __forceinline__ u32x4 ld16_any(const T* p) {
+    return *(const u32x4_any*)p;
 }
 
-// VEC consecutive elements, element i valid iff ok && i < nvalid
-template <typename T>
-__device__ __forceinline__ u32x4 ld_vec_checked(const T* p, bool ok, int nvalid, bool vec_ok) {
+// VEC elements of which element i is p[at(i)], zero unless i < nvalid; every
+// at(i) is a valid element, so there is no branch and the loads overlap
+template <typename T, typename At>
+__device__ __forceinline__ u32x4 ld16_each(const T* p, At at, int nvalid) {
     constexpr int VEC = Elem<T>::VEC;
-    if (ok && vec_ok && nvalid >= VEC) return *(const u32x4*)p;
-    uint32_t w[4] = {0u, 0u, 0u, 0u};
-    if (ok) {
-        if constexpr (sizeof(T) == 4) {
+    uint32_t x[VEC];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) w[i] = ld_bits(p + i, i < nvalid);
-        } else {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) w[i >> 1] |= ld_bits(p + i, i < nvalid) << (16 * (i & 1));
-        }
+    for (int i = 0; i < VEC; ++i) {
+        if constexpr (sizeof(T) == 4) x[i] = *(const uint32_t*)(p + at(i));
+        else x[i] = *(const uint16_t*)(p + at(i));
+        if (i >= nvalid) x[i] = 0u;
     }
-    return u32x4{w[0], w[1], w[2], w[3]};
+    if constexpr (sizeof(T) == 4) return u32x4{x[0], x[1], x[2], x[3]};
+    else return u32x4{x[0] | x[1] << 16, x[2] | x[3] << 16, x[4] | x[5] << 16, x[6] | x[7] << 16};
+}
+
+// elements s .. VEC - 1 of v moved down to 0 .. (s < VEC; the rest is zero)
+template <typename T>
+__device__ __forceinline__ u32x4 drop_elems(u32x4 v, int s) {
+    uint64_t lo = v[0] | (uint64_t)v[1] << 32, hi = v[2] | (uint64_t)v[3] << 32;
+    const int bits = s * 8 * (int)sizeof(T);
+    if (bits >= 64) { lo = hi; hi = 0; }
+    const int r = bits & 63;
+    if (r) {
+        lo = lo >> r | hi << (64 - r);
+        hi >>= r;
+    }
+    return u32x4{(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)};
 }
 
 // Row i of the transpose of a VEC x VEC block held as VEC vectors (one per k).
@@ -165,6 +175,13 @@ __device__ __forceinline__ u32x4 transpose_row(const u32x4* v, int i) {
 }
 
 // Global -> register -> LDS staging of one operand tile: R rows (m or n) x BK.
+// CHECKED: any edge and any alignment, without a branch per load (with one, each
+// load waited for the one before it: NT 2001 x 2003 x 2005 on this kernel fp32
+// 321 -> 156 us, fp16 227 -> 46; fp16 TN 347 -> 81). Rows past the matrix repeat its last row, a
+// block of VEC columns that crosses its edge is read VEC columns back from the
+// edge and moved into place when it is stored to LDS; what they leave in LDS
+// rows past the matrix only reaches results that are not stored. In the step
+// that crosses kend, elements are read one by one at clamped k and zero past it.
 template <typename T, int R, bool KMAJ, bool CHECKED>
 struct Stager {
     static constexpr int VEC = Elem<T>::VEC;
@@ -177,21 +194,25 @@ struct Stager {
 
     // base: operand pointer for this batch; row0: first m/n of the tile;
     // rows: M or N; k0: first k of this K step; kend: end of this K slice.
-    __device__ __forceinline__ void load(const T* base, int64_t ld, int row0, int rows, int k0,
-                                         int kend, bool vec_ok, int tid) {
+    __device__ __forceinline__ void load(const T* base, int64_t ld, int row0, int rows, int k0, int kend, int tid) {
+        if (!CHECKED || k0 + BK <= kend) load_step<false>(base, ld, row0, rows, k0, kend, tid);
+        else load_step<true>(base, ld, row0, rows, k0, kend, tid);
+    }
+
+    template <bool TAIL>
+    __device__ __forceinline__ void load_step(const T* base, int64_t ld, int row0, int rows, int k0, int kend,
+                                              int tid) {
         if constexpr (KMAJ) {
 #pragma unroll
             for (int i = 0; i < NV; ++i) {
                 const int c = tid + i * 256;
                 if (NCHUNK % 256 == 0 || c < NCHUNK) {
                     const int r = c >> 3, kc = c & 7;
-                    const int row = row0 + r, k = k0 + kc * VEC;
-                    const T* ptr = base + (int64_t)row * ld + k;
-                    if constexpr (!CHECKED) {
-                        v[i] = *(const u32x4*)ptr;
-                    } else {
-                        v[i] = ld_vec_checked<T>(ptr, row < rows, kend - k, vec_ok);
-                    }
+                    const int row = CHECKED ? min(row0 + r, rows - 1) : row0 + r, k = k0 + kc * VEC;
+                    const T* ptr = base + (int64_t)row * ld;
+                    if constexpr (!CHECKED) v[i] = *(const u32x4*)(ptr + k);
+                    else if constexpr (!TAIL) v[i] = ld16_any(ptr + k);
+                    else v[i] = ld16_each(ptr, [&](int e) { return min(k + e, kend - 1); }, kend - k);
                 }
             }
         } else {
@@ -204,11 +225,14 @@ struct Stager {
 #pragma unroll
                     for (int kk = 0; kk < VEC; ++kk) {
                         const int k = k0 + kb * VEC + kk;
-                        const T* ptr = base + (int64_t)k * ld + mn;
+                        const T* ptr = base + (int64_t)(TAIL ? min(k, kend - 1) : k) * ld;
+                        u32x4& d = v[j * VEC + kk];
                         if constexpr (!CHECKED) {
-                            v[j * VEC + kk] = *(const u32x4*)ptr;
+                            d = *(const u32x4*)(ptr + mn);
                         } else {
-                            v[j * VEC + kk] = ld_vec_checked<T>(ptr, k < kend, rows - mn, vec_ok);
+                            if (rows >= VEC) d = ld16_any(ptr + min(mn, rows - VEC));   // uniform
+                            else d = ld16_each(ptr, [&](int e) { return min(mn + e, rows - 1); }, VEC);
+                            if (TAIL && k >= kend) d = u32x4{0u, 0u, 0u, 0u};
                         }
                     }
                 }
@@ -216,7 +240,7 @@ struct Stager {
         }
     }
 
-    __device__ __forceinline__ void store(u32x4* tile, int tid) const {
+    __device__ __forceinline__ void store(u32x4* tile, int tid, int row0, int rows) {
         if constexpr (KMAJ) {
 #pragma unroll
             for (int i = 0; i < NV; ++i) {
@@ -227,6 +251,15 @@ struct Stager {
                 }
             }
         } else {
+            if (CHECKED && rows >= VEC && row0 + R > rows) {   // an edge tile: blocks read back from the edge
+#pragma unroll
+                for (int j = 0; j < NV / VEC; ++j) {
+                    const int mn = row0 + (tid + j * 256) % (R / VEC) * VEC;
+                    const int s = max(0, min(mn - (rows - VEC), VEC - 1));
+#pragma unroll
+                    for (int kk = 0; kk < VEC; ++kk) v[j * VEC + kk] = drop_elems<T>(v[j * VEC + kk], s);
+                }
+            }
 #pragma unroll
             for (int j = 0; j < NV / VEC; ++j) {
                 const int bi = tid + j * 256;
@@ -243,51 +276,26 @@ struct Stager {
     }
 };
 
-// Four results to C: fp32 as is, fp16 / bf16 rounded to nearest even.
+// Four results to C: fp32 as is, fp16 / bf16 rounded to nearest even; vec: the
+// address is aligned to the four elements (else to one).
 template <typename TC>
 __device__ __forceinline__ void store4(TC* p, const float* x, bool vec) {
-    if constexpr (sizeof(TC) == 4) {
-        if (vec) {
-            *(float4*)p = make_float4(x[0], x[1], x[2], x[3]);
-        } else {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) p[i] = x[i];
-        }
-    } else {
-        typedef TC v4 __attribute__((ext_vector_type(4)));
-        if (vec) {
-            v4 h;
-            h[0] = (TC)x[0]; h[1] = (TC)x[1];
-            h[2] = (TC)x[2]; h[3] = (TC)x[3];
-            *(v4*)p = h;
-        } else {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) p[i] = (TC)x[i];
-        }
-    }
+    typedef TC v4 __attribute__((ext_vector_type(4)));
+    typedef v4 v4_any __attribute__((aligned(2), may_alias));
+    v4 h;
+    h[0] = (TC)x[0]; h[1] = (TC)x[1];
+    h[2] = (TC)x[2]; h[3] = (TC)x[3];
+    if (vec) *(v4*)p = h;
+    else *(v4_any*)p = h;
 }
 
 template <typename TC>
 __device__ __forceinline__ void load4(const TC* p, float* x, bool vec) {
-    if constexpr (sizeof(TC) == 4) {
-        if (vec) {
-            float4 f = *(const float4*)p;
-            x[0] = f.x; x[1] = f.y; x[2] = f.z; x[3] = f.w;
-        } else {
+    typedef TC v4 __attribute__((ext_vector_type(4)));
+    typedef v4 v4_any __attribute__((aligned(2), may_alias));
+    const v4 h = vec ? *(const v4*)p : *(const v4_any*)p;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) x[i] = p[i];
-        }
-    } else {
-        typedef TC v4 __attribute__((ext_vector_type(4)));
-        if (vec) {
-            v4 h = *(const v4*)p;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) x[i] = (float)h[i];
-        } else {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) x[i] = (float)p[i];
-        }
-    }
+    for (int i = 0; i < 4; ++i) x[i] = (float)h[i];
 }
 
 // T: input element, TC: output element, AK: A is K-major (op_a == N),
@@ -326,15 +334,11 @@ __global__ __launch_bounds__(256) void gemm_kernel(KParams p) {
     const T* Bb;
     TC* Cb;
     const TC* Ci;   // beta's matrix (Cb itself in place)
-    bool va = p.vec_a != 0, vb = p.vec_b != 0, vc = p.vec_c != 0;
     if (p.ptr_array) {
         Ab = ((const T* const*)p.A)[b];
         Bb = ((const T* const*)p.B)[b];
         Cb = ((TC* const*)p.C)[b];
         Ci = Cb;
-        va = va && ((uintptr_t)Ab & 15) == 0;
-        vb = vb && ((uintptr_t)Bb & 15) == 0;
-        vc = vc && ((uintptr_t)Cb & (4 * sizeof(TC) - 1)) == 0;
     } else {
         Ab = (const T*)p.A + (int64_t)b * p.sa;
         Bb = (const T*)p.B + (int64_t)b * p.sb;
@@ -358,10 +362,10 @@ __global__ __launch_bounds__(256) void gemm_kernel(KParams p) {
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
     if (nkt > 0) {
-        sa.load(Ab, p.lda, m0, (int)p.M, kbeg, kend, va, tid);
-        sb.load(Bb, p.ldb, n0, (int)p.N, kbeg, kend, vb, tid);
-        sa.store(&lds[0][0], tid);
-        sb.store(&lds[0][BM * 8], tid);
+        sa.load(Ab, p.lda, m0, (int)p.M, kbeg, kend, tid);
+        sb.load(Bb, p.ldb, n0, (int)p.N, kbeg, kend, tid);
+        sa.store(&lds[0][0], tid, m0, (int)p.M);
+        sb.store(&lds[0][BM * 8], tid, n0, (int)p.N);
     }
     __syncthreads();
 
@@ -377,8 +381,8 @@ __global__ __launch_bounds__(256) void gemm_kernel(KParams p) {
         const bool more = kt + 1 < nkt;
         if (more) {
             const int k0 = kbeg + (kt + 1) * BK;
-            sa.load(Ab, p.lda, m0, (int)p.M, k0, kend, va, tid);
-            sb.load(Bb, p.ldb, n0, (int)p.N, k0, kend, vb, tid);
+            sa.load(Ab, p.lda, m0, (int)p.M, k0, kend, tid);
+            sb.load(Bb, p.ldb, n0, (int)p.N, k0, kend, tid);
         }
         const u32x4* As = &lds[cur][0];
         const u32x4* Bs = &lds[cur][BM * 8];
@@ -430,8 +434,8 @@ __global__ __launch_bounds__(256) void gemm_kernel(KParams p) {
             }
         }
         if (more) {
-            sa.store(&lds[cur ^ 1][0], tid);
-            sb.store(&lds[cur ^ 1][BM * 8], tid);
+            sa.store(&lds[cur ^ 1][0], tid, m0, (int)p.M);
+            sb.store(&lds[cur ^ 1][BM * 8], tid, n0, (int)p.N);
         }
         __syncthreads();
     }
@@ -467,12 +471,12 @@ __global__ __launch_bounds__(256) void gemm_kernel(KParams p) {
                     if (nv >= 4) {
                         if (beta != 0.0f) {
                             float o[4];
-                            load4<TC>(cirow + n, o, vc);
+                            load4<TC>(cirow + n, o, false);
 #pragma unroll
                             for (int e = 0; e < 4; ++e) x[e] += beta * o[e];
                         }
                         add_bias4(p.epi, n, 4, x);
-                        store4<TC>(crow + n, x, vc);
+                        store4<TC>(crow + n, x, false);
                     } else {
                         if (beta != 0.0f) {
 #pragma unroll
