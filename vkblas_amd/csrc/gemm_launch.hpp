@@ -259,6 +259,8 @@ static int launch_gemm_typed(const vkb_gemm_args* a, int tile, hipStream_t st) {
         // column N - BN on: whole 16-byte chunks need N % CV == 0 as well
         p.c_rows16 = !p.ptr_array && a->ldc % CV == 0 && aligned(a->C, 16) && (!multi || a->stride_c % CV == 0) &&
                      (p.split == 1 || p.s_split % CV == 0) && (a->N % bn == 0 || a->N % CV == 0);
+        p.cin_rows16 = !p.ptr_array && p.epi.ldcin % CV == 0 && aligned(p.epi.cin, 16) &&
+                       (!multi || p.epi.scin % CV == 0);
     }
     auto report = [&](int k) {
         if (a->kernel_out) *a->kernel_out = k;
@@ -300,8 +302,10 @@ static int launch_gemm_typed(const vkb_gemm_args* a, int tile, hipStream_t st) {
         //    tiles, 11.9 -> 10.9 against the direct one, 640 x 640, 100, 10.4 / 10.9);
         //    and instead of the pipelined 128x128 kernel on one wave of tiles
         //    where beta adds to C after at most 1024 k, as it reads C before the K
-        //    loop and not after it (bf16 -> fp32 TN, 4096 x 1024 x 512 13.2 -> 11.0 us,
-        //    1024 x 1024 x 512 10.9 -> 8.4, K = 1024 18.5 -> 17.8, but 2048 24.9 -> 26.2);
+        //    loop and not after it (us, pipelined / this: bf16 -> fp32 TN 4096 x 1024 x
+        //    512 13.5 / 12.5, 1024 x 1024 x 512 10.0 / 7.7, x 1024 13.1 / 10.8, 4096 x
+        //    1024 x 1024 level, fp16 NT 2000 x 1000 x 1024 11.9 / 10.8; at K = 2048
+        //    the pipelined kernel is ahead, 24.9 / 26.2 before its own row reads);
         //  * gemm_direct_kernel (small tiles, fragments straight from memory)
         //    - instead of the pipelined 128x128 kernel for fp32 on at most 128
         //      of its tiles, half the CUs (fp32 us, NT / NN / TN: 512 x 1024^2,

@@ -61,6 +61,7 @@ struct KParams {
     // batch stride and the split-K stride too): the pipelined kernel's
     // staged epilogue stores whole rows in 16-byte units
     int c_rows16;
+    int cin_rows16;   // the same of beta's matrix
     // Cin (beta's matrix) and the bias vector; vec_c covers Cin's alignment too
     EpiParams epi;
     // A, B, C are device arrays of `batch` matrix pointers (the sa / sb / sc

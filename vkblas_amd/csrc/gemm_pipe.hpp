@@ -582,6 +582,89 @@ __global__ __launch_bounds__(256, (WT == 128 || NST == 4) ? 1 : 2) void gemm_pip
     load_scalars(p, alpha, beta);
     constexpr int NQ = SH == 0 ? 1 : 4;
     const float beta_u = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, beta)));
+    if (beta_u != 0.0f && p.c_rows16 && p.cin_rows16) {
+        // beta's matrix read and C written as row segments, as in the staged
+        // form below, but alpha * acc staged in fp32 and beta's matrix added on
+        // read-out, LB loads of 16 bytes per lane at a time: the first round
+        // leaves before the staging, each later one before the stores of the
+        // round before it. Bound by C's traffic, with one workgroup per CU and
+        // nothing to overlap it; through the MFMA layout each load waited
+        // behind the store before it, which may alias it. Buffers new on each
+        // call, us, before and after: bf16 -> fp32 TN 11008 x 4096 x 8192 648 /
+        // 613, 4096 x 4096 x 1024 66 / 57, 8192 x 8192 x 1024 272 / 239; fp16 NT
+        // 4096 x 4096 x 1024 59 / 38; fp32 NN 263 / 250. (A 64 MB fp32 C left in
+        // the caches by the call before: 48 / 56 at 4096 x 4096 x 1024.) Loads and
+        // stores of one row group alternating (a rolling buffer) wait for the
+        // stores: 11008 x 4096 x 8192 673; rounds of 8 loads 621, of 16 606.
+        constexpr int CV = 16 / (int)sizeof(TC);             // elements of C per lane
+        constexpr int STR = WT * 4 + 16;                     // padded LDS row stride
+        constexpr int PROWS = WT == 128 ? 64 : WT;           // rows per pass
+        constexpr int LPR = WT / CV;                         // lanes per row on read-out
+        constexpr int RPI = 64 / LPR;                        // rows per instruction
+        constexpr int LB = PROWS / RPI < 16 ? PROWS / RPI : 16;
+        constexpr int ROUNDS = WT / RPI / LB;
+        static_assert(4 * PROWS * STR <= 2 * NST * STG * 16, "epilogue staging exceeds LDS");
+        typedef TC cvec __attribute__((ext_vector_type(CV)));
+        char* wl = (char*)lds + wave * (PROWS * STR);
+        const int c = lane % LPR * CV, n = n0 + wn * WT + c;
+        const int mrow = m0 + wm * WT + lane / LPR;
+        TC* cl = Cb + n;
+        const TC* cil = (const TC*)p.epi.cin + (sk ? 0 : (int64_t)b * p.epi.scin) + n;
+        // an edge tile stores what the tile before it does not (chunks start on n_lo)
+        auto mine = [&](int m) { return m >= m_lo && m < (int)p.M && n >= n_lo; };
+        cvec o[2][LB];
+        auto load_round = [&](int rd) {
+#pragma unroll
+            for (int k = 0; k < LB; ++k) {
+                const int m = mrow + (rd * LB + k) * RPI;
+                if (mine(m)) o[rd & 1][k] = __builtin_nontemporal_load((const cvec*)(cil + (int64_t)m * p.epi.ldcin));
+            }
+        };
+        load_round(0);
+        float bias[CV];
+#pragma unroll
+        for (int e = 0; e < CV; ++e) bias[e] = p.epi.bias ? bias_at(p.epi, n + e) : 0.0f;
+#pragma unroll
+        for (int rd = 0; rd < ROUNDS; ++rd) {
+            if (rd * LB * RPI % PROWS == 0) {                // the next PROWS rows of alpha * acc
+                const int r0 = rd * LB * RPI;
+                // a wave's LDS operations complete in order; the waits keep the
+                // compiler from reordering the cross-lane accesses
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+                for (int i = 0; i < NF; ++i) {
+                    if (i * FR < r0 || i * FR >= r0 + PROWS) continue;
+#pragma unroll
+                    for (int j = 0; j < NF; ++j)
+#pragma unroll
+                        for (int q = 0; q < NQ; ++q) {
+                            const int nl = j * FR + (SH == 0 ? 4 * (lane >> 4) : q * 8 + h * 4);
+                            float x[4];
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) x[e] = alpha * acc[i][j][q * 4 + e];
+                            store4<float>((float*)(wl + (i * FR + fl - r0) * STR + nl * 4), x, true);
+                        }
+                }
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            }
+            if (rd + 1 < ROUNDS) load_round(rd + 1);
+#pragma unroll
+            for (int k = 0; k < LB; ++k) {
+                const int r = (rd * LB + k) * RPI, m = mrow + r;
+                if (!mine(m)) continue;
+                cvec v;
+#pragma unroll
+                for (int q = 0; q < CV / 4; ++q) {
+                    const floatx4 x = *(const floatx4*)(wl + (r % PROWS + lane / LPR) * STR + (c + 4 * q) * 4);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        v[4 * q + e] = (TC)(x[e] + beta * (float)o[rd & 1][k][4 * q + e] + bias[4 * q + e]);
+                }
+                __builtin_nontemporal_store(v, (cvec*)(cl + (int64_t)m * p.ldc));
+            }
+        }
+        return;
+    }
     // bias of this lane's output columns, loaded once (inside the unrolled
     // store loops the per-element loads make them too large to unroll)
     const bool has_bias = p.epi.bias != nullptr;
