@@ -11,7 +11,8 @@ engine entry points (``vkblas_gemm_f32`` / ``vkblas_gemm_f16`` of the
 reference's ``src/vkblas.h:27-77``) with the same argument meaning and status
 codes.  There is no fallback: if the library is missing, loading raises.
 The asynchronous GEMMs go through ``_call`` (csrc/pycall.c), which converts
-their arguments natively; arguments it does not know go through ctypes.
+their arguments natively; arguments it does not know, and every call of an
+interpreter it is not built for, go through ctypes.
 """
 from __future__ import annotations
 
@@ -25,8 +26,6 @@ LIB_NAME = "libvkblas_hipblas.so"
 LIB_PATH = os.path.join(HERE, LIB_NAME)
 # the host dispatcher and kernels, opened by LIB_PATH's first call
 ENGINE_PATH = os.path.join(HERE, "libvkblas_engine.so")
-# the binding's calls (module vkblas_amd._call)
-CALL_PATH = os.path.join(HERE, "_call.so")
 
 # vkblas_status_t (reference src/vkblas.h:6-12)
 OK, ERR_INIT, ERR_IMPORT, ERR_PARAM, ERR_FALLBACK = 0, 1, 2, 3, 4
@@ -60,8 +59,12 @@ class Plan(ctypes.Structure):
                 ("k_per_split", ctypes.c_uint32), ("tail_rows", ctypes.c_uint32)]
 
 
+def _ctypes_call(*args):
+    return None
+
+
 _lib = None
-_native = None      # vkblas_amd._call.gemm_ex, set by load()
+_native = _ctypes_call      # vkblas_amd._call.gemm_ex where load() finds it
 _ex_addr = 0        # address of vkblas_gemm_ex_async
 
 _u32, _i64, _f, _vp, _int = ctypes.c_uint32, ctypes.c_int64, ctypes.c_float, ctypes.c_void_p, ctypes.c_int
@@ -78,7 +81,7 @@ def load():
     global _lib, _native, _ex_addr
     if _lib is not None:
         return _lib
-    for path in (LIB_PATH, ENGINE_PATH, CALL_PATH):
+    for path in (LIB_PATH, ENGINE_PATH):
         if not os.path.exists(path):
             raise RuntimeError(f"{path} is missing: run __graft_entry__.build() (make -C vkblas_amd)")
     L = ctypes.CDLL(LIB_PATH)
@@ -108,8 +111,12 @@ def load():
     L.vkblas_gemm_noalloc_async.argtypes = L.vkblas_gemm_async.argtypes
     L.vkblas_gemm_noalloc_async.restype = _int
     L.vkblas_noalloc_scratch_bytes.restype = ctypes.c_size_t
-    from . import _call
-    _native, _ex_addr = _call.gemm_ex, ctypes.cast(L.vkblas_gemm_ex_async, ctypes.c_void_p).value
+    try:
+        from ._call import gemm_ex
+    except ImportError:     # not built, or for another interpreter
+        pass
+    else:
+        _native, _ex_addr = gemm_ex, ctypes.cast(L.vkblas_gemm_ex_async, ctypes.c_void_p).value
     _lib = L
     return L
 
