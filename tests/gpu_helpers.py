@@ -14,6 +14,24 @@ from vkblas_amd import hipblas_abi as hb
 
 DEV = "cuda:0"
 
+# by type name: fp32 values -> the type's patterns (numpy) and back, the torch and engine types
+CONV = {"f32": lambda x: x, "f16": oracle.f2h_rne, "bf16": oracle.f2bf_rne}
+BACK = {"f32": lambda x: x, "f16": oracle.h2f, "bf16": oracle.bf2f}
+TORCH = {"f32": torch.float32, "f16": torch.float16, "bf16": torch.bfloat16}
+ENGINE = {"f32": vk.DT_F32, "f16": vk.DT_F16, "bf16": vk.DT_BF16}
+
+
+def to_dev_as(a: np.ndarray, dt: str) -> torch.Tensor:
+    """numpy (float32, or uint16 patterns of fp16 / bf16) -> device tensor of type dt."""
+    t = torch.from_numpy(a.view(np.int16) if a.dtype == np.uint16 else a).to(DEV)
+    return t.view(TORCH[dt]) if dt != "f32" else t
+
+
+def patterns(t: torch.Tensor) -> np.ndarray:
+    """device tensor -> numpy as CONV makes it"""
+    torch.cuda.synchronize()
+    return t.cpu().numpy() if t.dtype == torch.float32 else t.cpu().view(torch.int16).numpy().view(np.uint16)
+
 
 def to_dev(a: np.ndarray) -> torch.Tensor:
     """numpy (float32 or uint16 fp16 patterns) -> device tensor of the same bytes."""

@@ -9,12 +9,11 @@ import pytest
 import torch
 
 import oracle
+from gpu_helpers import (BACK, BF16_BOUND, CONV, ENGINE, F16_BOUND, f32_bound, normwise, patterns,
+                         to_dev_as as _dev)
 
 pytestmark = pytest.mark.gpu
 
-CONV = {"f32": lambda x: x, "f16": oracle.f2h_rne, "bf16": oracle.f2bf_rne}
-BACK = {"f32": lambda x: x, "f16": oracle.h2f, "bf16": oracle.bf2f}
-TD = {"f32": torch.float32, "f16": torch.float16, "bf16": torch.bfloat16}
 TYPES = [("f32", "f32"), ("f32", "f16"), ("f32", "bf16"), ("f16", "f16"), ("f16", "f32"), ("bf16", "bf16"),
          ("bf16", "f32")]
 # M, N, K, batch.  64 x 64 tiles from 144 of them on, else 32 x 32 (fp32 with
@@ -24,18 +23,12 @@ SHAPES = [(33, 32, 1, 1), (65, 47, 15, 1), (95, 33, 33, 2), (129, 65, 64, 3),   
           (65, 64, 257, 72), (129, 127, 511, 36), (193, 321, 1027, 7)]           # 64 x 64
 
 
-def _dev(a, dt):
-    t = torch.from_numpy(a.view(np.int16) if a.dtype == np.uint16 else a).to("cuda:0")
-    return t.view(TD[dt]) if dt != "f32" else t
-
-
 @pytest.mark.parametrize("form", ["plain", "apart"])
 @pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
 @pytest.mark.parametrize("op_a,op_b", [(0, 0), (0, 1), (1, 0), (1, 1)])
 @pytest.mark.parametrize("ab,ct", TYPES)
 def test_direct(ab, ct, op_a, op_b, shape, form):
     import vkblas_amd as vk
-    from gpu_helpers import normwise, f32_bound, F16_BOUND, BF16_BOUND
     M, N, K, batch = shape
     print(f"[case] direct {ab}>{ct} op={op_a}{op_b} {shape} {form}", flush=True)
     r = np.random.default_rng(M + 3 * N + 7 * K + batch)
@@ -66,7 +59,7 @@ def test_direct(ab, ct, op_a, op_b, shape, form):
                                np.ascontiguousarray(b[1 + i * sb:][:ldb * rb]), ldb, alpha, beta, src, ldc, out, ldc,
                                BACK[ab](bias))
         want[1 + i * sc:][:ldc * M] = out
-    dt = {"f32": vk.DT_F32, "f16": vk.DT_F16, "bf16": vk.DT_BF16}
+    dt = ENGINE
     dA, dB, dC, dI, dBias = _dev(a, ab), _dev(b, ab), _dev(c0, ct), _dev(cin, ct), _dev(bias, ab)
     ea, ec = dA.element_size(), dC.element_size()
     vk.gemm_ex_async(dt[ab], dt[ct], op_a, op_b, M, N, K, alpha, dA.data_ptr() + ea, lda, dB.data_ptr() + ea, ldb,
@@ -75,7 +68,7 @@ def test_direct(ab, ct, op_a, op_b, shape, form):
                      stride_c_in=sc if form == "apart" else 0, bias=dBias.data_ptr(), bias_type=dt[ab])
     torch.cuda.synchronize()
     assert vk.last_kernel() == vk.KERNEL_DIRECT, vk.last_kernel()
-    got = dC.cpu().view(torch.int16).numpy().view(np.uint16) if ct != "f32" else dC.cpu().numpy()
+    got = patterns(dC)
     bound = BF16_BOUND if ct == "bf16" else F16_BOUND if "f16" in (ab, ct) or ab == "bf16" else f32_bound(K)
     for i in range(batch):
         g = BACK[ct](got[1 + i * sc:][:ldc * M]).reshape(M, ldc)

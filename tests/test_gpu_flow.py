@@ -9,12 +9,11 @@ import pytest
 import torch
 
 import oracle
+from gpu_helpers import (BACK, BF16_BOUND, CONV, ENGINE, F16_BOUND, f32_bound, normwise, patterns,
+                         to_dev_as as _dev)
 
 pytestmark = pytest.mark.gpu
 
-CONV = {"f32": lambda x: x, "f16": oracle.f2h_rne, "bf16": oracle.f2bf_rne}
-BACK = {"f32": lambda x: x, "f16": oracle.h2f, "bf16": oracle.bf2f}
-TD = {"f32": torch.float32, "f16": torch.float16, "bf16": torch.bfloat16}
 # M, N, K, batch (an MN-major operand's M or N is rounded up to a multiple of 8,
 # K to one of 8 unless both are MN-major):
 SHAPES = [(257, 63, 65, 40), (129, 127, 191, 40),      # 128 x 64 tiles: N of one, few of 128 x 128
@@ -23,18 +22,12 @@ SHAPES = [(257, 63, 65, 40), (129, 127, 191, 40),      # 128 x 64 tiles: N of on
           (257, 255, 72, 72), (130, 257, 200, 50)]     # two stages
 
 
-def _dev(a, dt):
-    t = torch.from_numpy(a.view(np.int16) if a.dtype == np.uint16 else a).to("cuda:0")
-    return t.view(TD[dt]) if dt != "f32" else t
-
-
 @pytest.mark.parametrize("form", ["plain", "apart"])
 @pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
 @pytest.mark.parametrize("op_a,op_b", [(0, 0), (0, 1), (1, 0), (1, 1)])
 @pytest.mark.parametrize("ab,ct", [("f16", "f16"), ("f16", "f32"), ("bf16", "bf16"), ("bf16", "f32")])
 def test_flow(ab, ct, op_a, op_b, shape, form):
     import vkblas_amd as vk
-    from gpu_helpers import normwise, F16_BOUND, BF16_BOUND
     M, N, K, batch = shape
     M, N = (-(-M // 8) * 8 if op_a else M), (N if op_b else -(-N // 8) * 8)
     K = K if op_a and not op_b else -(-K // 8) * 8
@@ -70,7 +63,7 @@ def test_flow(ab, ct, op_a, op_b, shape, form):
                                np.ascontiguousarray(b[i * sb:][:ldb * rb]), ldb, alpha, beta, src, ldc, out, ldc,
                                BACK[ab](bias), rows=rows)
         want[1 + i * sc:][:ldc * M] = out
-    dt = {"f32": vk.DT_F32, "f16": vk.DT_F16, "bf16": vk.DT_BF16}
+    dt = ENGINE
     dA, dB, dC, dI, dBias = _dev(a, ab), _dev(b, ab), _dev(c0, ct), _dev(cin, ct), _dev(bias, ab)
     ec = dC.element_size()
     vk.gemm_ex_async(dt[ab], dt[ct], op_a, op_b, M, N, K, alpha, dA.data_ptr(), lda, dB.data_ptr(), ldb,
@@ -79,7 +72,7 @@ def test_flow(ab, ct, op_a, op_b, shape, form):
                      stride_c_in=sc if form == "apart" else 0, bias=dBias.data_ptr(), bias_type=dt[ab])
     torch.cuda.synchronize()
     assert vk.last_kernel() == vk.KERNEL_FLOW, vk.last_kernel()
-    got = dC.cpu().view(torch.int16).numpy().view(np.uint16) if ct != "f32" else dC.cpu().numpy()
+    got = patterns(dC)
     first = c0.view(np.uint8).reshape(-1)
     for i in range(batch):
         g = got[1 + i * sc:][:ldc * M].reshape(M, ldc)

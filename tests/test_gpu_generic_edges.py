@@ -8,12 +8,11 @@ import pytest
 import torch
 
 import oracle
+from gpu_helpers import (BACK, BF16_BOUND, CONV, ENGINE, F16_BOUND, f32_bound, normwise, patterns,
+                         to_dev_as as _dev)
 
 pytestmark = pytest.mark.gpu
 
-CONV = {"f32": lambda x: x, "f16": oracle.f2h_rne, "bf16": oracle.f2bf_rne}
-BACK = {"f32": lambda x: x, "f16": oracle.h2f, "bf16": oracle.bf2f}
-TD = {"f32": torch.float32, "f16": torch.float16, "bf16": torch.bfloat16}
 # tile override (0: 64 x 64, 1: 128 x 128, 2: 256 x 256), M, N, K
 SHAPES = [(0, 3, 5, 1), (0, 65, 63, 31), (0, 9, 129, 65), (1, 129, 127, 63), (1, 2, 131, 33), (1, 250, 7, 100),
           (2, 257, 255, 67)]
@@ -26,17 +25,11 @@ def reset_override():
     vk.set_override(-1, False)
 
 
-def _dev(a, dt):
-    t = torch.from_numpy(a.view(np.int16) if a.dtype == np.uint16 else a).to("cuda:0")
-    return t.view(TD[dt]) if dt != "f32" else t
-
-
 @pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
 @pytest.mark.parametrize("op_a,op_b", [(0, 0), (0, 1), (1, 0), (1, 1)])
 @pytest.mark.parametrize("ab,ct", [("f32", "f32"), ("f16", "f16"), ("f16", "f32"), ("bf16", "bf16"), ("bf16", "f32")])
 def test_generic_edges(ab, ct, op_a, op_b, shape):
     import vkblas_amd as vk
-    from gpu_helpers import normwise, f32_bound, F16_BOUND, BF16_BOUND
     tile, M, N, K = shape
     print(f"[case] generic {ab}>{ct} op={op_a}{op_b} {shape}", flush=True)
     r = np.random.default_rng(M + 3 * N + 7 * K)
@@ -53,14 +46,14 @@ def test_generic_edges(ab, ct, op_a, op_b, shape):
     want = c[1:].copy()
     oracle.ref_gemm_epi_rm(ab, ct, op_a, op_b, M, N, K, a[1:].copy(), lda, b[1:].copy(), ldb, 1.25, -0.5, want.copy(),
                            ldc, want, ldc, None)
-    dt = {"f32": vk.DT_F32, "f16": vk.DT_F16, "bf16": vk.DT_BF16}
+    dt = ENGINE
     dA, dB, dC = _dev(a, ab), _dev(b, ab), _dev(c, ct)
     vk.set_override(tile, True)
     vk.gemm_async(dt[ab], dt[ct], op_a, op_b, M, N, K, 1.25, dA.data_ptr() + dA.element_size(), lda,
                   dB.data_ptr() + dB.element_size(), ldb, -0.5, dC.data_ptr() + dC.element_size(), ldc, split_k=1)
     torch.cuda.synchronize()
     assert vk.last_kernel() == vk.KERNEL_GENERIC_CHECKED, vk.last_kernel()
-    got = dC.cpu().view(torch.int16).numpy().view(np.uint16) if ct != "f32" else dC.cpu().numpy()
+    got = patterns(dC)
     assert np.array_equal(got[:1], c[:1]), "the element in front of C written"
     g, w = (BACK[ct](np.ascontiguousarray(x)).reshape(M, ldc) for x in (got[1:], want))
     assert np.array_equal(g[:, N:], w[:, N:]), "C padding written"

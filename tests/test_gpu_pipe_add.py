@@ -7,12 +7,11 @@ import pytest
 import torch
 
 import oracle
+from gpu_helpers import (BACK, BF16_BOUND, CONV, ENGINE, F16_BOUND, f32_bound, normwise, patterns,
+                         to_dev_as as _dev)
 
 pytestmark = pytest.mark.gpu
 
-CONV = {"f32": lambda x: x, "f16": oracle.f2h_rne, "bf16": oracle.f2bf_rne}
-BACK = {"f32": lambda x: x, "f16": oracle.h2f, "bf16": oracle.bf2f}
-TD = {"f32": torch.float32, "f16": torch.float16, "bf16": torch.bfloat16}
 # tile override (1: 128 x 128, 2: 256 x 256), M, N, K
 SHAPES = [(2, 512, 256, 256), (2, 264, 520, 256), (1, 128, 256, 256), (1, 200, 264, 256)]
 
@@ -24,18 +23,12 @@ def reset_override():
     vk.set_override(-1, False)
 
 
-def _dev(a, dt):
-    t = torch.from_numpy(a.view(np.int16) if a.dtype == np.uint16 else a).to("cuda:0")
-    return t.view(TD[dt]) if dt != "f32" else t
-
-
 @pytest.mark.parametrize("form", ["in_place", "apart", "apart_unaligned"])
 @pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
 @pytest.mark.parametrize("op_a,op_b", [(0, 1), (1, 0)])
 @pytest.mark.parametrize("ab,ct", [("f32", "f32"), ("f16", "f16"), ("f16", "f32"), ("bf16", "bf16"), ("bf16", "f32")])
 def test_add(ab, ct, op_a, op_b, shape, form):
     import vkblas_amd as vk
-    from gpu_helpers import normwise, f32_bound, F16_BOUND, BF16_BOUND
     tile, M, N, K = shape
     print(f"[case] pipe add {ab}>{ct} op={op_a}{op_b} {shape} {form}", flush=True)
     r = np.random.default_rng(M + 3 * N)
@@ -49,7 +42,7 @@ def test_add(ab, ct, op_a, op_b, shape, form):
     src, lds = (c.copy(), ldc) if form == "in_place" else (cin[off:off + M * ldi].copy(), ldi)
     want = c.copy()
     oracle.ref_gemm_epi_rm(ab, ct, op_a, op_b, M, N, K, a, lda, b, ldb, 1.25, -0.5, src, lds, want, ldc, BACK[ab](bias))
-    dt = {"f32": vk.DT_F32, "f16": vk.DT_F16, "bf16": vk.DT_BF16}
+    dt = ENGINE
     dA, dB, dC, dI, dBias = _dev(a, ab), _dev(b, ab), _dev(c, ct), _dev(cin, ct), _dev(bias, ab)
     vk.set_override(tile, False)
     vk.gemm_ex_async(dt[ab], dt[ct], op_a, op_b, M, N, K, 1.25, dA.data_ptr(), lda, dB.data_ptr(), ldb, -0.5,
@@ -58,7 +51,7 @@ def test_add(ab, ct, op_a, op_b, shape, form):
     torch.cuda.synchronize()
     if form != "apart_unaligned" or ct != "f32":   # fp32 off 16 bytes goes to the generic kernel
         assert vk.last_kernel() in (vk.KERNEL_PIPE256, vk.KERNEL_PIPE128, vk.KERNEL_PIPE128_4), vk.last_kernel()
-    got = dC.cpu().view(torch.int16).numpy().view(np.uint16) if ct != "f32" else dC.cpu().numpy()
+    got = patterns(dC)
     g, w = (BACK[ct](x).reshape(M, ldc) for x in (got, want))
     assert np.array_equal(g[:, N:], w[:, N:]), "C padding written"
     bound = BF16_BOUND if ct == "bf16" else f32_bound(K) if ab == "f32" else F16_BOUND
