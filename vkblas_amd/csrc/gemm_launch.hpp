@@ -40,6 +40,10 @@ static int launch_layout(const KParams& p, bool ak, bool bk, bool checked, uint3
 
 static inline bool aligned(const void* ptr, uintptr_t a) { return ((uintptr_t)ptr % a) == 0; }
 
+// Whether a launch can hold that many workgroups: HIP counts its threads in 32
+// bits, and past them runs a few workgroups and reports success.
+static inline bool launches(uint64_t workgroups, uint32_t threads) { return workgroups <= 0xffffffffull / threads; }
+
 // Compute units of the current device (cached per device; 0 if unknown).
 static inline uint32_t cu_count() {
     static int cached[64];
@@ -121,7 +125,7 @@ static int launch_flow(const vkb_gemm_args* a, KParams p, bool ak, bool bk, hipS
         const bool narrow = a->N <= 64 || t <= 128;
         if (narrow) p.tiles_n = (a->N + 63) / 64;
         const uint64_t grid = (uint64_t)p.tiles_m * p.tiles_n * mats;
-        if (grid == 0 || grid > 0x7fffffffull) return (int)hipErrorInvalidValue;
+        if (grid == 0 || !launches(grid, t <= 256 && !narrow ? 512 : 256)) return (int)hipErrorInvalidValue;
         const bool early = a->scalar_mode == VKB_SCALAR_HOST && a->beta != 0.0f;   // beta's matrix before the K loop
         if (narrow && early) return launch_flow_one<T, TC, 64, 3, 4, true>(p, ak, bk, (uint32_t)grid, st);
         if (narrow) return launch_flow_one<T, TC, 64, 3, 4>(p, ak, bk, (uint32_t)grid, st);
@@ -142,7 +146,8 @@ static int launch_flow(const vkb_gemm_args* a, KParams p, bool ak, bool bk, hipS
 //   tiles of 32) 25.1 / 12.0 / 8.2, 384^2 x 2048 (144) TN 37.8 / 16.9 / 20.0;
 //   fp16 NT 512^2 x 1024 11.9 / 8.4, 512 x 1024 x 1024 11.9 / 10.7, 768^3 10.4 / 12.1.
 // Returns 0 if no tile fits the operands (an MN-major operand needs a whole
-// tile in its dimension; a tile's rows must span less than 2^31 bytes).
+// tile in its dimension; a tile's rows must span less than 2^31 bytes) or the
+// launch: the larger tiles of the generic kernel then may.
 template <typename T>
 static uint32_t direct_tile(const vkb_gemm_args* a, uint64_t mats) {
     auto tiles = [&](uint32_t tm, uint32_t tn) {
@@ -153,6 +158,7 @@ static uint32_t direct_tile(const vkb_gemm_args* a, uint64_t mats) {
         // of an MN-major one
         const uint64_t ra = a->a_kmajor ? tm : 32, rb = a->b_kmajor ? tn : 32;
         return (a->a_kmajor || a->M >= tm) && (a->b_kmajor || a->N >= tn) &&
+               launches(tiles(tm, tn), 256) &&
                (ra * (uint64_t)a->lda + 64) * sizeof(T) < (1ull << 31) &&
                (rb * (uint64_t)a->ldb + 64) * sizeof(T) < (1ull << 31);
     };
@@ -187,7 +193,7 @@ static int launch_direct(const vkb_gemm_args* a, KParams p, uint32_t tile, bool 
     p.tiles_m = (a->M + tm - 1) / tm;
     p.tiles_n = (a->N + tn - 1) / tn;
     const uint64_t grid = (uint64_t)p.tiles_m * p.tiles_n * p.batch * p.split;
-    if (grid == 0 || grid > 0x7fffffffull) return (int)hipErrorInvalidValue;
+    if (grid == 0 || !launches(grid, 256)) return (int)hipErrorInvalidValue;
     if (tile == 64) return launch_direct_one<T, TC, 4, 4, 4>(p, ak, bk, (uint32_t)grid, st);
     if (tile == 32) return launch_direct_one<T, TC, 2, 2, 8>(p, ak, bk, (uint32_t)grid, st);
     if constexpr (sizeof(T) == 4) return launch_direct_one<T, TC, 1, 2, 8>(p, ak, bk, (uint32_t)grid, st);
@@ -270,7 +276,7 @@ static int launch_gemm_typed(const vkb_gemm_args* a, int tile, hipStream_t st) {
     const bool full = !p.ptr_array && (a->M % bm == 0) && (a->N % bn == 0) && (a->K % BK == 0) &&
                       p.vec_a && p.vec_b && p.vec_c;
     const uint64_t grid64 = (uint64_t)p.tiles_m * p.tiles_n * p.batch * p.split * p.nq;
-    if (grid64 == 0 || grid64 > 0x7fffffffull) return (int)hipErrorInvalidValue;
+    if (grid64 == 0 || !launches(grid64, 256)) return (int)hipErrorInvalidValue;
     const uint32_t grid = (uint32_t)grid64;
     const bool ak = a->a_kmajor != 0, bk = a->b_kmajor != 0;
     {

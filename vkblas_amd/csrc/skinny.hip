@@ -1258,6 +1258,10 @@ int launch_skh(const SkParams& p, float* part, uint32_t nsplit, hipStream_t st) 
 extern "C" uint32_t vkb_skinny_plan(int ab_type, int b_kmajor, uint32_t M, uint32_t N, uint32_t K, int64_t lda,
                                    int64_t ldb) {
     if (M == 0 || N == 0 || K == 0 || lda <= 0 || ldb <= 0) return 0;
+    // HIP counts a launch's threads in 32 bits, and past them runs a few
+    // workgroups and reports success: the GEMV takes 64 threads per weight row,
+    // the others at most 16 per weight row or column
+    if (N >= (M == 1 && b_kmajor && ab_type != VKB_T_F32 ? 1u << 26 : 1u << 28)) return 0;
     const int64_t es = ab_type == VKB_T_F32 ? 4 : 2;
     const int64_t vec = 16 / es;
     if ((M > 1 && (lda % vec || lda < (int64_t)K)) || ldb % vec) return 0;
