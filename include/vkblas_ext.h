@@ -39,7 +39,8 @@ typedef enum {
     VKBLAS_PATH_TILE128 = 2,  /* blocked MFMA GEMM, 128 x 128 tiles        */
     VKBLAS_PATH_TILE256 = 3,  /* blocked MFMA GEMM, 256 x 256 tiles        */
     VKBLAS_PATH_SPLITK = 4,   /* split-K pass 1 + deterministic reduce     */
-    VKBLAS_PATH_SKINNY = 5,   /* bandwidth-bound decode (M <= 64)          */
+    VKBLAS_PATH_SKINNY = 5,   /* bandwidth-bound decode (M <= 64); small
+                                 ones run VKBLAS_KERNEL_DIRECT             */
     VKBLAS_PATH_TAIL = 6      /* whole waves of tiles, then split-K over
                                  the last tail_rows rows of C             */
 } vkblas_path_t;
@@ -53,7 +54,7 @@ typedef enum {
     VKBLAS_KERNEL_PIPE256 = 3,          /* pipelined kernel, 256 x 256 tiles       */
     VKBLAS_KERNEL_PIPE128 = 4,          /* pipelined kernel, 128 x 128, 2 stages   */
     VKBLAS_KERNEL_PIPE128_4 = 5,        /* pipelined kernel, 128 x 128, 4 stages   */
-    VKBLAS_KERNEL_SKINNY = 6,           /* decode plans (vkblas_last_path skinny)  */
+    VKBLAS_KERNEL_SKINNY = 6,           /* decode kernels                          */
     VKBLAS_KERNEL_WAVEK = 7,            /* split-K pass 1 on 32 x 32 / 64 x 64
                                            tiles, the slice's K over the waves  */
     VKBLAS_KERNEL_DIRECT = 8,           /* small tiles, K over the waves, MFMA

@@ -19,6 +19,20 @@ pytestmark = pytest.mark.gpu
 NAN16 = np.uint16(0x7E00)     # quiet NaN, fp16 encoding
 NAN_BF16 = np.uint16(0x7FC0)  # quiet NaN, bf16 encoding
 
+ALLOWED = []   # the kernels that a case may run on, set by the fixture
+
+
+@pytest.fixture(autouse=True, params=["decode", "dispatched"])
+def kernels(request):
+    """Every case on the decode kernels themselves (a tile override keeps the small
+    decode plans from gemm_direct_kernel), and as it is dispatched."""
+    import vkblas_amd as vk
+    vk.set_override(0 if request.param == "decode" else -1, False)
+    ALLOWED[:] = [vk.KERNEL_SKINNY] + ([vk.KERNEL_DIRECT] if request.param == "dispatched" else [])
+    yield
+    vk.set_override(-1, False)
+
+
 CASES = []
 for M in (1, 2, 3, 4, 5, 8, 16):
     for (N, K) in ((1, 8), (7, 504), (100, 520), (1000, 1032), (300, 4104), (64, 8192)):
@@ -129,7 +143,7 @@ def test_decode_edges(case):
     ab = vk.DT_BF16 if bf else vk.DT_F16
     vk.gemm_async(ab, vk.DT_F32 if f32 else ab, vk.OP_N, vk.OP_T, M, N, K, 1.5, dX.data_ptr(), lda,
                   dW.data_ptr(), ldb, beta, dC.data_ptr(), ldc, stream=torch.cuda.current_stream().cuda_stream)
-    assert vk.last_path() == vk.PATH_SKINNY
+    assert vk.last_path() == vk.PATH_SKINNY and vk.last_kernel() in ALLOWED, vk.last_kernel()
     got = to_host(dC)
     if f32:
         g, w = got, want
@@ -158,7 +172,7 @@ def test_decode_device_scalars(M):
     vk.gemm_async(vk.DT_F16, vk.DT_F16, vk.OP_N, vk.OP_T, M, N, K, 0.0, dX.data_ptr(), K, dW.data_ptr(), K, 0.0,
                   dC.data_ptr(), N, scalar_mode=vk.SCALAR_DEV_F32, alpha_dev=sc.data_ptr(),
                   beta_dev=sc.data_ptr() + 4, stream=torch.cuda.current_stream().cuda_stream)
-    assert vk.last_path() == vk.PATH_SKINNY
+    assert vk.last_path() == vk.PATH_SKINNY and vk.last_kernel() in ALLOWED, vk.last_kernel()
     assert normwise(oracle.h2f(to_host(dC)), oracle.h2f(want)) <= F16_BOUND
 
 
@@ -239,7 +253,7 @@ def test_decode_kn(case):
     assert pl.path == vk.PATH_SKINNY, pl.path
     vk.gemm_async(ab, vk.DT_F32 if f32 else ab, vk.OP_N, vk.OP_N, M, N, K, 1.5, dX.data_ptr(), lda,
                   dW.data_ptr(), ldb, beta, dC.data_ptr(), ldc, stream=torch.cuda.current_stream().cuda_stream)
-    assert vk.last_path() == vk.PATH_SKINNY
+    assert vk.last_path() == vk.PATH_SKINNY and vk.last_kernel() in ALLOWED, vk.last_kernel()
     got = to_host(dC)
     if f32:
         g, w = got, want
@@ -272,7 +286,7 @@ def test_decode_kn_epilogue(M, N, K, sep):
     vk.gemm_ex_async(vk.DT_F16, vk.DT_F16, vk.OP_N, vk.OP_N, M, N, K, 1.25, dX.data_ptr(), K, dW.data_ptr(), N,
                      -0.5, dC.data_ptr(), N, c_in=dCin.data_ptr() if sep else None, ldc_in=N if sep else 0,
                      bias=dB.data_ptr(), bias_type=vk.DT_F32, stream=torch.cuda.current_stream().cuda_stream)
-    assert vk.last_path() == vk.PATH_SKINNY
+    assert vk.last_path() == vk.PATH_SKINNY and vk.last_kernel() in ALLOWED, vk.last_kernel()
     assert normwise(oracle.h2f(to_host(dC)), oracle.h2f(want)) <= F16_BOUND
 
 
@@ -289,6 +303,6 @@ def test_decode_kn_deterministic():
             dC = torch.empty(M * N, dtype=torch.float16, device="cuda:0")
             vk.gemm_async(vk.DT_F16, vk.DT_F16, vk.OP_N, vk.OP_N, M, N, K, 1.0, dX.data_ptr(), K, dW.data_ptr(), N,
                           0.0, dC.data_ptr(), N, stream=torch.cuda.current_stream().cuda_stream)
-            assert vk.last_path() == vk.PATH_SKINNY
+            assert vk.last_path() == vk.PATH_SKINNY and vk.last_kernel() in ALLOWED, vk.last_kernel()
             outs.append(to_host(dC))
         assert all(np.array_equal(outs[0], o) for o in outs[1:])

@@ -27,6 +27,19 @@ pytestmark = pytest.mark.gpu
 
 SENT = np.float32(-7.25)   # value of C's padding columns, checked afterwards
 
+ALLOWED = []   # the kernels that a case may run on, set by the fixture
+
+
+@pytest.fixture(autouse=True, params=["decode", "dispatched"])
+def kernels(request):
+    """Every case on the decode kernels themselves (a tile override keeps the small
+    decode plans from gemm_direct_kernel), and as it is dispatched."""
+    import vkblas_amd as vk
+    vk.set_override(0 if request.param == "decode" else -1, False)
+    ALLOWED[:] = [vk.KERNEL_SKINNY] + ([vk.KERNEL_DIRECT] if request.param == "dispatched" else [])
+    yield
+    vk.set_override(-1, False)
+
 # (M, N, K, pad_a, pad_b, pad_c, beta): lda = K + pad_a and ldb = K + pad_b
 # (N x K) or N + pad_b (K x N) are multiples of 4 (lda may be anything for M = 1)
 CASES_T = []
@@ -131,7 +144,7 @@ def _run(case, op_b, ex=None):
                          ldc_in=ldc if dCin is not None else 0, bias=dBias.data_ptr(), bias_type=vk.DT_F32,
                          stream=st)
     assert vk.last_path() == vk.PATH_SKINNY
-    assert vk.last_kernel() == vk.KERNEL_SKINNY
+    assert vk.last_kernel() in ALLOWED, vk.last_kernel()
     got = to_host(dC).reshape(M, ldc)
     w = want.reshape(M, ldc)
     assert np.array_equal(got[:, N:], w[:, N:]), "C padding written"
@@ -194,7 +207,7 @@ def test_skinny_f32_device_scalars(op_b, M):
     vk.gemm_async(vk.DT_F32, vk.DT_F32, vk.OP_N, op_b, M, N, K, 0.0, dX.data_ptr(), K, dW.data_ptr(), ldb, 0.0,
                   dC.data_ptr(), N, scalar_mode=vk.SCALAR_DEV_F32, alpha_dev=sc.data_ptr(),
                   beta_dev=sc.data_ptr() + 4, stream=torch.cuda.current_stream().cuda_stream)
-    assert vk.last_path() == vk.PATH_SKINNY
+    assert vk.last_path() == vk.PATH_SKINNY and vk.last_kernel() in ALLOWED
     assert normwise(to_host(dC), want) <= f32_bound(K)
 
 
@@ -216,6 +229,6 @@ def test_skinny_f32_deterministic():
             dC = torch.empty(M * N, dtype=torch.float32, device="cuda:0")
             vk.gemm_async(vk.DT_F32, vk.DT_F32, vk.OP_N, op_b, M, N, K, 1.0, dX.data_ptr(), K, dW.data_ptr(), ldb,
                           0.0, dC.data_ptr(), N, stream=torch.cuda.current_stream().cuda_stream)
-            assert vk.last_path() == vk.PATH_SKINNY
+            assert vk.last_path() == vk.PATH_SKINNY and vk.last_kernel() in ALLOWED
             outs.append(to_host(dC))
         assert all(np.array_equal(outs[0], o) for o in outs[1:])

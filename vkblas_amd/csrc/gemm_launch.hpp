@@ -345,8 +345,7 @@ static int launch_gemm_typed(const vkb_gemm_args* a, int tile, hipStream_t st) {
                                          ((uint64_t)klen * sizeof(T) >= 512 || t64 <= 512);
             const uint32_t dt = want ? direct_tile<T>(a, mats) : 0;
             if (dt) {
-                // a decode plan's call still reports a decode kernel
-                report(a->direct == 2 ? VKB_KERN_SKINNY : VKB_KERN_DIRECT);
+                report(VKB_KERN_DIRECT);
                 return launch_direct<T, TC>(a, p, dt, ak, bk, st);
             }
         }
