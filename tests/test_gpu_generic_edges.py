@@ -13,9 +13,12 @@ from gpu_helpers import (BACK, BF16_BOUND, CONV, ENGINE, F16_BOUND, f32_bound, n
 
 pytestmark = pytest.mark.gpu
 
-# tile override (0: 64 x 64, 1: 128 x 128, 2: 256 x 256), M, N, K
-SHAPES = [(0, 3, 5, 1), (0, 65, 63, 31), (0, 9, 129, 65), (1, 129, 127, 63), (1, 2, 131, 33), (1, 250, 7, 100),
-          (2, 257, 255, 67)]
+# tile override (0: 64 x 64, 1: 128 x 128, 2: 256 x 256), M, N, K, split
+SHAPES = [(0, 3, 5, 1, 1), (0, 65, 63, 31, 1), (0, 9, 129, 65, 1), (1, 129, 127, 63, 1), (1, 2, 131, 33, 1),
+          (1, 250, 7, 100, 1), (2, 257, 255, 67, 1),
+          (0, 5, 3, 300, 1), (1, 131, 2, 129, 1), (0, 70, 6, 7, 1),       # fewer than a vector along M, N, K
+          # slices of whole K steps, the last one shorter than a vector (fp16 64 + 64 + 5, fp32 4 x 32 + 5)
+          (0, 65, 63, 133, 5), (1, 129, 3, 133, 5)]
 
 
 @pytest.fixture(autouse=True)
@@ -30,7 +33,7 @@ def reset_override():
 @pytest.mark.parametrize("ab,ct", [("f32", "f32"), ("f16", "f16"), ("f16", "f32"), ("bf16", "bf16"), ("bf16", "f32")])
 def test_generic_edges(ab, ct, op_a, op_b, shape):
     import vkblas_amd as vk
-    tile, M, N, K = shape
+    tile, M, N, K, split = shape
     print(f"[case] generic {ab}>{ct} op={op_a}{op_b} {shape}", flush=True)
     r = np.random.default_rng(M + 3 * N + 7 * K)
     ra, ca = (K, M) if op_a else (M, K)
@@ -50,7 +53,7 @@ def test_generic_edges(ab, ct, op_a, op_b, shape):
     dA, dB, dC = _dev(a, ab), _dev(b, ab), _dev(c, ct)
     vk.set_override(tile, True)
     vk.gemm_async(dt[ab], dt[ct], op_a, op_b, M, N, K, 1.25, dA.data_ptr() + dA.element_size(), lda,
-                  dB.data_ptr() + dB.element_size(), ldb, -0.5, dC.data_ptr() + dC.element_size(), ldc, split_k=1)
+                  dB.data_ptr() + dB.element_size(), ldb, -0.5, dC.data_ptr() + dC.element_size(), ldc, split_k=split)
     torch.cuda.synchronize()
     assert vk.last_kernel() == vk.KERNEL_GENERIC_CHECKED, vk.last_kernel()
     got = patterns(dC)

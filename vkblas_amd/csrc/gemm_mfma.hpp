@@ -144,6 +144,27 @@ __device__ __forceinline__ u32x4 ld16_each(const T* p, At at, int nvalid) {
     else return u32x4{x[0] | x[1] << 16, x[2] | x[3] << 16, x[4] | x[5] << 16, x[6] | x[7] << 16};
 }
 
+// the first n of VEC elements (n < VEC, the same in every lane); the others are
+// zero (16-bit) or the n-th (32-bit: no branch, the loads overlap)
+template <typename T>
+__device__ __forceinline__ u32x4 ld16_first(const T* p, int n) {
+    u32x4 d;
+    if constexpr (sizeof(T) == 4) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) d[i] = *(const uint32_t*)(p + min(i, n - 1));
+    } else {
+        uint32_t x[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            x[i] = 0u;
+            if (i < n) x[i] = *(const uint16_t*)(p + i);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) d[i] = x[2 * i] | x[2 * i + 1] << 16;
+    }
+    return d;
+}
+
 // elements s .. VEC - 1 of v moved down to 0 .. (s < VEC; the rest is zero)
 template <typename T>
 __device__ __forceinline__ u32x4 drop_elems(u32x4 v, int s) {
@@ -176,13 +197,19 @@ __device__ __forceinline__ u32x4 transpose_row(const u32x4* v, int i) {
 }
 
 // Global -> register -> LDS staging of one operand tile: R rows (m or n) x BK.
-// CHECKED: any edge and any alignment, without a branch per load (with one, each
-// load waited for the one before it: NT 2001 x 2003 x 2005 on this kernel fp32
-// 321 -> 156 us, fp16 227 -> 46; fp16 TN 347 -> 81). Rows past the matrix repeat its last row, a
-// block of VEC columns that crosses its edge is read VEC columns back from the
-// edge and moved into place when it is stored to LDS; what they leave in LDS
-// rows past the matrix only reaches results that are not stored. In the step
-// that crosses kend, elements are read one by one at clamped k and zero past it.
+// CHECKED: any edge and any alignment. load() has no branch around single loads
+// (with one, each waited for the one before it: NT 2001 x 2003 x 2005 on this
+// kernel fp32 321 -> 156 us, fp16 227 -> 46; fp16 TN 347 -> 81) and nothing that
+// needs a loaded value: rows past the matrix repeat its last row, blocks of
+// columns outside it load nothing (their LDS rows only reach results that are not
+// stored) and one that crosses its edge is read VEC columns back from it. place()
+// does the rest, where the loads have come back in any case: it moves those blocks
+// into place, zeroes k rows past the end, and reads by itself, element by element,
+// what load() leaves out: the step that crosses the end of a K-major operand and
+// an MN-major one of fewer than VEC columns (narrow). With the other order, a choice
+// between two ways to load in load(), each load waited (us, that / this, before
+// either: f32 TN 4 of 119 x 10 x 15684 1416 / 628, 963; NN 64 of 5 x 24 x 6100 392 /
+// 190, 303; pointer arrays TN 4 of 64 x 64 x 2440 131 / 81, 115).
 template <typename T, int R, bool KMAJ, bool CHECKED>
 struct Stager {
     static constexpr int VEC = Elem<T>::VEC;
@@ -192,56 +219,85 @@ struct Stager {
     static constexpr int NBLK = 8 * (R / VEC);
     static constexpr int NV = KMAJ ? (NCHUNK + 255) / 256 : ((NBLK + 255) / 256) * VEC;
     u32x4 v[NV];
+    const T* base;      // operand of this batch
+    int64_t ld;
+    int row0, rows;     // first m / n of the tile; M or N
+    int kend;           // end of this K slice
+    int tid;
 
-    // base: operand pointer for this batch; row0: first m/n of the tile;
-    // rows: M or N; k0: first k of this K step; kend: end of this K slice.
-    __device__ __forceinline__ void load(const T* base, int64_t ld, int row0, int rows, int k0, int kend, int tid) {
-        if (!CHECKED || k0 + BK <= kend) load_step<false>(base, ld, row0, rows, k0, kend, tid);
-        else load_step<true>(base, ld, row0, rows, k0, kend, tid);
-    }
+    __device__ __forceinline__ bool narrow() const { return CHECKED && rows < VEC; }
 
-    template <bool TAIL>
-    __device__ __forceinline__ void load_step(const T* base, int64_t ld, int row0, int rows, int k0, int kend,
-                                              int tid) {
+    // the loads of the K step from k0 on
+    __device__ __forceinline__ void load(int k0) {
         if constexpr (KMAJ) {
+            if (CHECKED && k0 + BK > kend) return;
 #pragma unroll
             for (int i = 0; i < NV; ++i) {
-                const int c = tid + i * 256;
+                const int c = tid + i * 256, k = k0 + (c & 7) * VEC;
                 if (NCHUNK % 256 == 0 || c < NCHUNK) {
-                    const int r = c >> 3, kc = c & 7;
-                    const int row = CHECKED ? min(row0 + r, rows - 1) : row0 + r, k = k0 + kc * VEC;
-                    const T* ptr = base + (int64_t)row * ld;
-                    if constexpr (!CHECKED) v[i] = *(const u32x4*)(ptr + k);
-                    else if constexpr (!TAIL) v[i] = ld16_any(ptr + k);
-                    else v[i] = ld16_each(ptr, [&](int e) { return min(k + e, kend - 1); }, kend - k);
+                    if constexpr (!CHECKED) v[i] = *(const u32x4*)(base + (int64_t)(row0 + (c >> 3)) * ld + k);
+                    else v[i] = ld16_any(base + (int64_t)min(row0 + (c >> 3), rows - 1) * ld + k);
                 }
             }
         } else {
+            const int end = narrow() ? 0 : rows;    // in the lanes' condition: no branch of its own
 #pragma unroll
             for (int j = 0; j < NV / VEC; ++j) {
                 const int bi = tid + j * 256;
-                if (NBLK % 256 == 0 || bi < NBLK) {
-                    const int kb = bi / (R / VEC), mb = bi % (R / VEC);
-                    const int mn = row0 + mb * VEC;
+                const int kb = bi / (R / VEC), mn = row0 + bi % (R / VEC) * VEC;
+                if ((NBLK % 256 == 0 || bi < NBLK) & (!CHECKED || ((mn < end) & (k0 + kb * VEC < kend)))) {
 #pragma unroll
                     for (int kk = 0; kk < VEC; ++kk) {
                         const int k = k0 + kb * VEC + kk;
-                        const T* ptr = base + (int64_t)(TAIL ? min(k, kend - 1) : k) * ld;
-                        u32x4& d = v[j * VEC + kk];
-                        if constexpr (!CHECKED) {
-                            d = *(const u32x4*)(ptr + mn);
-                        } else {
-                            if (rows >= VEC) d = ld16_any(ptr + min(mn, rows - VEC));   // uniform
-                            else d = ld16_each(ptr, [&](int e) { return min(mn + e, rows - 1); }, VEC);
-                            if (TAIL && k >= kend) d = u32x4{0u, 0u, 0u, 0u};
-                        }
+                        const T* ptr = base + (int64_t)(CHECKED ? min(k, kend - 1) : k) * ld;
+                        if constexpr (!CHECKED) v[j * VEC + kk] = *(const u32x4*)(ptr + mn);
+                        else v[j * VEC + kk] = ld16_any(ptr + min(mn, rows - VEC));
                     }
                 }
             }
         }
     }
 
-    __device__ __forceinline__ void store(u32x4* tile, int tid, int row0, int rows) {
+    // the vectors of the step from k0 on as the tile has them
+    __device__ __forceinline__ void place(int k0) {
+        const bool tail = k0 + BK > kend;
+        if constexpr (KMAJ) {
+            if (!tail) return;
+#pragma unroll
+            for (int i = 0; i < NV; ++i) {
+                const int c = tid + i * 256, row = row0 + (c >> 3), k = k0 + (c & 7) * VEC;
+                v[i] = u32x4{0u, 0u, 0u, 0u};
+                if (row < rows && k < kend)
+                    v[i] = ld16_each(base + (int64_t)row * ld, [&](int e) { return min(k + e, kend - 1); }, kend - k);
+            }
+        } else if (narrow()) {              // one tile, its first blocks
+#pragma unroll
+            for (int j = 0; j < NV / VEC; ++j) {
+                const int bi = tid + j * 256, k = k0 + bi / (R / VEC) * VEC;
+#pragma unroll
+                for (int kk = 0; kk < VEC; ++kk) {
+                    v[j * VEC + kk] = u32x4{0u, 0u, 0u, 0u};
+                    if (k0 + kk < kend && bi % (R / VEC) == 0 && k + kk < kend)
+                        v[j * VEC + kk] = ld16_first(base + (int64_t)(k + kk) * ld, rows);
+                }
+            }
+        } else {
+            if (!tail && row0 + R <= rows) return;
+#pragma unroll
+            for (int j = 0; j < NV / VEC; ++j) {
+                const int bi = tid + j * 256, k = k0 + bi / (R / VEC) * VEC;
+                const int s = max(0, min(row0 + bi % (R / VEC) * VEC - (rows - VEC), VEC - 1));
+#pragma unroll
+                for (int kk = 0; kk < VEC; ++kk) {
+                    v[j * VEC + kk] = drop_elems<T>(v[j * VEC + kk], s);
+                    if (k + kk >= kend) v[j * VEC + kk] = u32x4{0u, 0u, 0u, 0u};
+                }
+            }
+        }
+    }
+
+    // the step from k0 on, loaded and placed before, to LDS
+    __device__ __forceinline__ void store(u32x4* tile) const {
         if constexpr (KMAJ) {
 #pragma unroll
             for (int i = 0; i < NV; ++i) {
@@ -252,15 +308,6 @@ struct Stager {
                 }
             }
         } else {
-            if (CHECKED && rows >= VEC && row0 + R > rows) {   // an edge tile: blocks read back from the edge
-#pragma unroll
-                for (int j = 0; j < NV / VEC; ++j) {
-                    const int mn = row0 + (tid + j * 256) % (R / VEC) * VEC;
-                    const int s = max(0, min(mn - (rows - VEC), VEC - 1));
-#pragma unroll
-                    for (int kk = 0; kk < VEC; ++kk) v[j * VEC + kk] = drop_elems<T>(v[j * VEC + kk], s);
-                }
-            }
 #pragma unroll
             for (int j = 0; j < NV / VEC; ++j) {
                 const int bi = tid + j * 256;
@@ -362,11 +409,17 @@ __global__ __launch_bounds__(256) void gemm_kernel(KParams p) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
+    sa.base = Ab; sa.ld = p.lda; sa.row0 = m0; sa.rows = (int)p.M; sa.kend = kend; sa.tid = tid;
+    sb.base = Bb; sb.ld = p.ldb; sb.row0 = n0; sb.rows = (int)p.N; sb.kend = kend; sb.tid = tid;
     if (nkt > 0) {
-        sa.load(Ab, p.lda, m0, (int)p.M, kbeg, kend, tid);
-        sb.load(Bb, p.ldb, n0, (int)p.N, kbeg, kend, tid);
-        sa.store(&lds[0][0], tid, m0, (int)p.M);
-        sb.store(&lds[0][BM * 8], tid, n0, (int)p.N);
+        sa.load(kbeg);
+        sb.load(kbeg);
+        if (CHECKED) {
+            sa.place(kbeg);
+            sb.place(kbeg);
+        }
+        sa.store(&lds[0][0]);
+        sb.store(&lds[0][BM * 8]);
     }
     __syncthreads();
 
@@ -380,10 +433,14 @@ __global__ __launch_bounds__(256) void gemm_kernel(KParams p) {
     for (int kt = 0; kt < nkt; ++kt) {
         const int cur = kt & 1;
         const bool more = kt + 1 < nkt;
+        const int k0 = kbeg + (kt + 1) * BK;
+        // the loads before are in LDS: nothing is waited for, but the compiler,
+        // which sees lanes that load and do not store, waits here and not
+        // between the loads below (vmcnt 0, the other counters untouched)
+        if (CHECKED) __builtin_amdgcn_s_waitcnt(0x0f70);
         if (more) {
-            const int k0 = kbeg + (kt + 1) * BK;
-            sa.load(Ab, p.lda, m0, (int)p.M, k0, kend, tid);
-            sb.load(Bb, p.ldb, n0, (int)p.N, k0, kend, tid);
+            sa.load(k0);
+            sb.load(k0);
         }
         const u32x4* As = &lds[cur][0];
         const u32x4* Bs = &lds[cur][BM * 8];
@@ -435,8 +492,12 @@ __global__ __launch_bounds__(256) void gemm_kernel(KParams p) {
             }
         }
         if (more) {
-            sa.store(&lds[cur ^ 1][0], tid, m0, (int)p.M);
-            sb.store(&lds[cur ^ 1][BM * 8], tid, n0, (int)p.N);
+            if (CHECKED) {
+                sa.place(k0);
+                sb.place(k0);
+            }
+            sa.store(&lds[cur ^ 1][0]);
+            sb.store(&lds[cur ^ 1][BM * 8]);
         }
         __syncthreads();
     }
