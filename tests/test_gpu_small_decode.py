@@ -1,4 +1,4 @@
-"""Decode plans on either side of the line between gemm_direct_kernel and the decode
+"""Decode plans on either side of the lines between gemm_direct_kernel and the decode
 kernels: vkblas_last_kernel names the kernel that ran, vkblas_last_path stays the
 plan's, and the result agrees with the CPU oracle."""
 import numpy as np
@@ -18,6 +18,16 @@ CASES = [
     ("f32", 1, 20, 28, 13, False), ("f16", 0, 8, 24, 64, False),        # fewer than 32 columns
     ("f16", 1, 40, 1000, 2056, False), ("f16", 0, 40, 1000, 2056, False),   # K past 2048
     ("f32", 0, 16, 4096, 260, False), ("bf16", 1, 64, 8192, 520, False),    # weight past the line
+]
+# the lines in N (8192, 16-bit K x N 16384), in K (fp32 1280), in tiles (16-bit N x K) and
+# of one or two rows
+LINES = [
+    ("f32", 1, 17, 8192, 8, True), ("f32", 1, 17, 8200, 8, False), ("f32", 0, 4, 8192, 16, True),
+    ("f32", 0, 4, 8200, 16, False), ("f16", 1, 20, 8192, 16, True), ("f16", 1, 20, 8200, 16, False),
+    ("f16", 0, 2, 16384, 24, True), ("f16", 0, 2, 16392, 24, False), ("bf16", 0, 8, 42616, 32, False),
+    ("f32", 1, 33, 96, 1280, True), ("f32", 1, 33, 96, 1284, False), ("f32", 0, 16, 40, 1284, False),
+    ("f16", 1, 33, 4096, 520, True), ("f16", 1, 33, 4104, 520, False), ("f16", 1, 33, 4104, 512, True),
+    ("f32", 0, 2, 256, 32, False), ("f32", 0, 2, 256, 36, True), ("f32", 0, 3, 256, 32, True),
 ]
 
 
@@ -43,7 +53,7 @@ def _run(ab, op_b, M, N, K, lda, ldb, kernel):
     assert normwise(BACK[ab](patterns(dC)), BACK[ab](want)) <= bound
 
 
-@pytest.mark.parametrize("case", CASES, ids=lambda c: "{}_op{}_{}x{}x{}_{}".format(*c))
+@pytest.mark.parametrize("case", CASES + LINES, ids=lambda c: "{}_op{}_{}x{}x{}_{}".format(*c))
 def test_kernel_and_result(case):
     import vkblas_amd as vk
     ab, op_b, M, N, K, direct = case

@@ -704,11 +704,24 @@ static void prof_end(prof_t* pf, hipStream_t stream, const char* what, int ok) {
  *   fp16 NT, 17-64 rows: 1024^2 10.9-11.8 / 8.4-8.6, 2048^2 11.5 / 9.6-10.9,
  *   512 x 4096 10.9-12.3 / 11.4-12.5; NN, 1-64 rows: 2048^2 11.0-13.9 / 8.8-10.6,
  *   512 x 4096 11.3 / 11.3.
- * Up to 16 rows against N x K the decode kernels are level or ahead. */
+ * Up to 16 rows against N x K the decode kernels are level or ahead.  So they
+ * are (us of GPU time, 1500 calls of random sizes)
+ *   where N alone is large and the tiles many: from N = 8192 on, fp16 K x N
+ *   from 16384 (fp32 NT 17 x 12264 x 64 3.5 / 4.7, NN 1 x 9392 x 16 2.8 / 3.9, 1 x
+ *   52168 x 16 3.2 / 7.1; fp16 NT 20 x 17784 x 16 4.8 / 8.0, NN 2 x 19440 x 24 3.7 /
+ *   6.1, 2 x 59080 x 24 3.8 / 10.8; 4 x 12032 x 56 4.5 / 3.7);
+ *   fp32 past K = 1280, where four waves share too long a K on few tiles (NT 48
+ *   x 96 x 1920 10.8 / 13.5, 20 x 440 x 1776 9.0 / 10.8; NN 32 x 40 x 1896 8.7 / 9.7);
+ *   fp32 K x N, one or two rows and at most 32 k (1 x 6888 x 8 3.0 / 3.4);
+ *   fp16 NT past K = 512 where the tiles of 32 x 32 are more than the CUs (33 x
+ *   5576 x 640, 350 tiles, 5.6 / 7.2; 64 x 4088 x 856, 256, 9.3 / 5.8; 64 x 6272 x
+ *   352, 392, 7.3 / 4.1). */
 static int small_decode(vkblas_dtype_t ab_type, vkblas_op_t op_b, uint32_t M, uint32_t N, uint32_t K) {
-    const uint64_t most = ab_type == VKBLAS_DT_F32 ? 1ull << 20 : 1ull << 22;
-    return g_force_tile < 0 && !g_generic_only && (M >= 17 || op_b == VKBLAS_OP_N) && N >= 32 && K <= 2048 &&
-           (uint64_t)N * K <= most;
+    const int f32 = ab_type == VKBLAS_DT_F32, kn = op_b == VKBLAS_OP_N;
+    return g_force_tile < 0 && !g_generic_only && (M >= 17 || kn) && N >= 32 &&
+           N <= (kn && !f32 ? 16384u : 8192u) && K <= (f32 ? 1280u : 2048u) && !(f32 && kn && M <= 2 && K <= 32) &&
+           (f32 || kn || K <= 512 || ((M + 31) / 32) * ((N + 31) / 32) <= 256) &&
+           (uint64_t)N * K <= (f32 ? 1ull << 20 : 1ull << 22);
 }
 
 /* The body of vkblas_gemm_async.  ws_ext != NULL: the split-K / decode
