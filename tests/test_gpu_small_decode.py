@@ -60,3 +60,14 @@ def test_kernel_and_result(case):
     print(f"[case] small decode {case}", flush=True)
     _run(ab, op_b, M, N, K, K + -K % 8, (K if op_b else N) + -(K if op_b else N) % 8,
          vk.KERNEL_DIRECT if direct else vk.KERNEL_SKINNY)
+
+
+@pytest.mark.parametrize("ab,op_b,M,N,K,lda,ldb", [
+    ("f16", 0, 3, 64, 64, 1 << 25, 64),         # the last token of each of three sequences of 8192 x 4096
+    ("f32", 0, 3, 64, 64, 1 << 24, 64), ("f32", 0, 2, 64, 40, 40, 1 << 24),
+    ("bf16", 1, 17, 64, 64, 1 << 25, 64)])
+def test_rows_gigabytes_apart(ab, op_b, M, N, K, lda, ldb):
+    """Leading dimensions past gemm_direct_kernel's 32-bit offsets: the decode kernels'."""
+    import vkblas_amd as vk
+    print(f"[case] small decode, far rows {ab} op_b={op_b} {M}x{N}x{K} lda={lda} ldb={ldb}", flush=True)
+    _run(ab, op_b, M, N, K, lda, ldb, vk.KERNEL_SKINNY)

@@ -715,10 +715,14 @@ static void prof_end(prof_t* pf, hipStream_t stream, const char* what, int ok) {
  *   fp32 K x N, one or two rows and at most 32 k (1 x 6888 x 8 3.0 / 3.4);
  *   fp16 NT past K = 512 where the tiles of 32 x 32 are more than the CUs (33 x
  *   5576 x 640, 350 tiles, 5.6 / 7.2; 64 x 4088 x 856, 256, 9.3 / 5.8; 64 x 6272 x
- *   352, 392, 7.3 / 4.1). */
-static int small_decode(vkblas_dtype_t ab_type, vkblas_op_t op_b, uint32_t M, uint32_t N, uint32_t K) {
+ *   352, 392, 7.3 / 4.1).
+ * They keep leading dimensions of which 64 rows span 2 GiB (the last token of
+ * each of a few long sequences): gemm_direct_kernel's offsets are 32-bit. */
+static int small_decode(vkblas_dtype_t ab_type, vkblas_op_t op_b, uint32_t M, uint32_t N, uint32_t K, uint32_t lda,
+                        uint32_t ldb) {
     const int f32 = ab_type == VKBLAS_DT_F32, kn = op_b == VKBLAS_OP_N;
-    return g_force_tile < 0 && !g_generic_only && (M >= 17 || kn) && N >= 32 &&
+    const uint64_t span = 65ull * (lda > ldb ? lda : ldb) * (f32 ? 4 : 2);
+    return span < 1ull << 31 && g_force_tile < 0 && !g_generic_only && (M >= 17 || kn) && N >= 32 &&
            N <= (kn && !f32 ? 16384u : 8192u) && K <= (f32 ? 1280u : 2048u) && !(f32 && kn && M <= 2 && K <= 32) &&
            (f32 || kn || K <= 512 || ((M + 31) / 32) * ((N + 31) / 32) <= 256) &&
            (uint64_t)N * K <= (f32 ? 1ull << 20 : 1ull << 22);
@@ -776,7 +780,7 @@ static vkblas_status_t gemm_impl(vkblas_dtype_t ab_type, vkblas_dtype_t c_type, 
      * partials: [split][M][N] fp32 for split-K and the split decode kernel,
      * [split][tail_rows][N] for the split tail; with divided K slices
      * (VKB_TILE_64Q) then the parts' sums, VKB_WAVEK_NQ x the partials */
-    const int direct = plan.path == VKBLAS_PATH_SKINNY && small_decode(ab_type, op_b, M, N, K);
+    const int direct = plan.path == VKBLAS_PATH_SKINNY && small_decode(ab_type, op_b, M, N, K, lda, ldb);
     if (direct && plan.split > 1 && !ws_ext) {
         /* a decode plan with a K split is refused under stream capture
          * whatever kernel would run it, as ws_acquire refuses it */
