@@ -76,3 +76,30 @@ def test_direct(ab, ct, op_a, op_b, shape, form):
         assert np.array_equal(g[:, N:], w[:, N:]), "C padding written"
         assert np.all(np.isfinite(g[:, :N]))
         assert normwise(g[:, :N], w[:, :N]) <= bound, i
+
+
+# type, op_a, op_b, M, N, K, batch, kernel: both sides of the lines in tiles of 64 x 64
+@pytest.mark.parametrize("ab,op_a,op_b,M,N,K,batch,kernel", [
+    ("f32", 0, 1, 576, 64, 320, 15, "DIRECT"), ("f32", 0, 1, 576, 64, 320, 16, "GENERIC"),      # whole tiles, NT: 144
+    ("f16", 0, 1, 320, 192, 192, 6, "DIRECT"), ("f16", 0, 1, 256, 384, 192, 4, "GENERIC"),      # 16 bits: 96
+    ("f32", 1, 0, 640, 64, 128, 16, "DIRECT"), ("f32", 1, 0, 768, 64, 128, 16, "GENERIC"),      # others: 192
+    ("f32", 1, 0, 448, 64, 64, 20, "DIRECT"), ("f32", 1, 0, 576, 64, 64, 16, "GENERIC"),        # a short K: 144
+    # edges, K below 512 bytes: 256 tiles
+    ("f16", 1, 1, 343, 13, 5, 42, "DIRECT"), ("f16", 1, 1, 343, 13, 5, 43, "GENERIC_CHECKED"),
+    ("f32", 0, 0, 7, 509, 127, 32, "DIRECT"), ("f32", 0, 0, 7, 509, 127, 33, "GENERIC_CHECKED"),
+    ("f32", 0, 0, 7, 509, 128, 33, "DIRECT")])
+def test_line_against_the_generic_kernel(ab, op_a, op_b, M, N, K, batch, kernel):
+    import vkblas_amd as vk
+    print(f"[case] line {ab} op={op_a}{op_b} {M}x{N}x{K} x{batch}", flush=True)
+    r = np.random.default_rng(M + 3 * N + 7 * K)
+    lda, ldb = (M if op_a else K), (K if op_b else N)
+    a, b = (CONV[ab](r.uniform(-1, 1, batch * n).astype(np.float32)) for n in (M * K, N * K))
+    want = CONV[ab](np.zeros(M * N, np.float32))
+    oracle.ref_gemm_epi_rm(ab, ab, op_a, op_b, M, N, K, a[-M * K:].copy(), lda, b[-N * K:].copy(), ldb, 1.25, 0.0,
+                           want.copy(), N, want, N, None)
+    dA, dB, dC = _dev(a, ab), _dev(b, ab), _dev(CONV[ab](np.zeros(batch * M * N, np.float32)), ab)
+    vk.gemm_async(ENGINE[ab], ENGINE[ab], op_a, op_b, M, N, K, 1.25, dA.data_ptr(), lda, dB.data_ptr(), ldb, 0.0,
+                  dC.data_ptr(), N, batch=batch, stride_a=M * K, stride_b=N * K, stride_c=M * N)
+    assert vk.last_kernel() == getattr(vk, "KERNEL_" + kernel), vk.last_kernel()
+    got = patterns(dC)[-M * N:].copy()
+    assert normwise(BACK[ab](got), BACK[ab](want)) <= (f32_bound(K) if ab == "f32" else F16_BOUND)

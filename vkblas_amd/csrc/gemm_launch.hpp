@@ -320,11 +320,17 @@ static int launch_gemm_typed(const vkb_gemm_args* a, int tile, hipStream_t st) {
         //      89 against 122 / 102 / 85).  16-bit inputs stay there: level at
         //      32 tiles, ahead from 36 on (768 x 1024 x 3072 fp16 22 against 26);
         //    - instead of the generic kernel with edge handling, but not where
-        //      direct_loses (many tiles) or for many tiles with a short K, where
-        //      the four waves have too little to share (96 x 197 x 197 x 64 fp16
-        //      9.8 against 15.0);
+        //      direct_loses (many tiles) or past 256 tiles with a short K, where
+        //      the four waves have too little to share (of random calls with K below
+        //      512 bytes 4 of 283 lost up to 128 tiles, 6 of 57 up to 256, 25 of 49
+        //      up to 512; fp16 TT 64 of 343 x 13 x 5, 384 tiles, 6.5 -> 7.7);
         //    - instead of the generic kernel on whole tiles where 64 x 64 ones
-        //      would leave CUs idle (fp32 NT 512^2 x 2048 49 -> 25).
+        //      would leave CUs idle (fp32 NT 512^2 x 2048 49 -> 25): with both
+        //      operands along K, where the generic kernel has nothing to
+        //      transpose, below 144 tiles in fp32 (128 tiles 8.4 -> 6.8, 144 73 ->
+        //      83) and 96 in 16 bits (64 tiles 3.5 -> 3.0, 96 13.7 -> 16.8), else
+        //      below 192 (fp16 TN 176, K = 1216, 22 -> 10), 144 for a short K
+        //      (fp32 TN 160, K = 64, 5.1 -> 5.5).
         if (a->direct && !p.ptr_array && !a->generic_only &&
             (tile == VKB_TILE_64 || tile == VKB_TILE_128 || tile == VKB_TILE_256) &&
             !(tile == VKB_TILE_64 && p.split > 1 && full)) {
@@ -340,9 +346,9 @@ static int launch_gemm_typed(const vkb_gemm_args* a, int tile, hipStream_t st) {
             const uint32_t klen = p.split > 1 ? p.kps : a->K;
             const bool want = a->direct == 2 ? true
                             : pipe ? sizeof(T) == 4 && tile == VKB_TILE_128 && p.split == 1 && grid <= 128
-                            : full ? t64 < 192
+                            : full ? t64 < (ak && bk ? (sizeof(T) == 4 ? 144u : 96u) : klen * sizeof(T) >= 512 ? 192u : 144u)
                                    : !direct_loses<T>(ak, bk, t64, klen) &&
-                                         ((uint64_t)klen * sizeof(T) >= 512 || t64 <= 512);
+                                         ((uint64_t)klen * sizeof(T) >= 512 || t64 <= 256);
             const uint32_t dt = want ? direct_tile<T>(a, mats) : 0;
             if (dt) {
                 report(VKB_KERN_DIRECT);
