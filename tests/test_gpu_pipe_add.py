@@ -56,3 +56,27 @@ def test_add(ab, ct, op_a, op_b, shape, form):
     assert np.array_equal(g[:, N:], w[:, N:]), "C padding written"
     bound = BF16_BOUND if ct == "bf16" else f32_bound(K) if ab == "f32" else F16_BOUND
     assert normwise(g[:, :N], w[:, :N]) <= bound
+
+
+@pytest.mark.parametrize("K", [1024, 16512])
+def test_add_large(K):
+    """an fp32 C of 64 MiB that is stored to stay in the caches, and past them where the
+    operands of the call drive it out (in all more than 320 MiB)"""
+    import vkblas_amd as vk
+    M = N = 4096
+    print(f"[case] pipe add {M}x{N}x{K}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(K)
+    a, b = (torch.randn(K, 4096, device="cuda", generator=g).bfloat16() for _ in range(2))
+    c = torch.randn(M, N, device="cuda", generator=g)
+    rows = oracle.sample_rows(M, 8)
+    want = c.cpu().numpy().reshape(-1)
+    hc = want.copy()
+    oracle.ref_gemm_epi_rm("bf16", "f32", 1, 0, M, N, K, patterns(a).reshape(-1), M, patterns(b).reshape(-1), N, 1.25, -0.5,
+                           hc, N, want, N, None, rows=rows)
+    vk.set_override(2, False)
+    vk.gemm_async(vk.DT_BF16, vk.DT_F32, 1, 0, M, N, K, 1.25, a.data_ptr(), M, b.data_ptr(), N, -0.5, c.data_ptr(), N,
+                  split_k=1)
+    assert vk.last_kernel() == vk.KERNEL_PIPE256, vk.last_kernel()
+    got = patterns(c)
+    assert np.all(np.isfinite(got))
+    assert normwise(got[rows], want.reshape(M, N)[rows]) <= F16_BOUND

@@ -265,6 +265,11 @@ static int launch_gemm_typed(const vkb_gemm_args* a, int tile, hipStream_t st) {
         // column N - BN on: whole 16-byte chunks need N % CV == 0 as well
         p.c_rows16 = !p.ptr_array && a->ldc % CV == 0 && aligned(a->C, 16) && (!multi || a->stride_c % CV == 0) &&
                      (p.split == 1 || p.s_split % CV == 0) && (a->N % bn == 0 || a->N % CV == 0);
+        // the operands and C together near the 256 MiB of the Infinity Cache or
+        // below: past 320 MiB storing C past the caches is level or ahead for
+        // the same C on each call too (8192 x 8192 x 2048, 320 MiB, 315 / 320 us)
+        p.c_stays = p.batch * (((uint64_t)a->M + a->N) * a->K * sizeof(T) + (uint64_t)a->M * a->N * sizeof(TC)) <=
+                    (320ull << 20);
         p.cin_rows16 = !p.ptr_array && p.epi.ldcin % CV == 0 && aligned(p.epi.cin, 16) &&
                        (!multi || p.epi.scin % CV == 0);
     }

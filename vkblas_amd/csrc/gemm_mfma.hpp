@@ -62,6 +62,7 @@ struct KParams {
     // staged epilogue stores whole rows in 16-byte units
     int c_rows16;
     int cin_rows16;   // the same of beta's matrix
+    int c_stays;      // C may still be in the caches when the next call adds to it
     // Cin (beta's matrix) and the bias vector; vec_c covers Cin's alignment too
     EpiParams epi;
     // A, B, C are device arrays of `batch` matrix pointers (the sa / sb / sc

@@ -591,11 +591,20 @@ __global__ __launch_bounds__(256, (WT == 128 || NST == 4) ? 1 : 2) void gemm_pip
         // nothing to overlap it; through the MFMA layout each load waited
         // behind the store before it, which may alias it. Buffers new on each
         // call, us, before and after: bf16 -> fp32 TN 11008 x 4096 x 8192 648 /
-        // 613, 4096 x 4096 x 1024 66 / 57, 8192 x 8192 x 1024 272 / 239; fp16 NT
-        // 4096 x 4096 x 1024 59 / 38; fp32 NN 263 / 250. (A 64 MB fp32 C left in
-        // the caches by the call before: 48 / 56 at 4096 x 4096 x 1024.) Loads and
+        // 613, fp16 -> fp32 4096 x 4096 x 1024 65 / 61, 8192 x 8192 x 1024 273 /
+        // 249, fp16 NT 4096 x 4096 x 1024 59 / 38; fp32 NN 261 / 251. Loads and
         // stores of one row group alternating (a rolling buffer) wait for the
         // stores: 11008 x 4096 x 8192 673; rounds of 8 loads 621, of 16 606.
+        // A program that adds to one fp32 C call after call finds it in the
+        // caches, unless the call's own traffic drives it out (c_stays): stored
+        // past them, each call read it from memory (the same C on each call,
+        // fp16 -> fp32 TN, MFMA layout / non-temporal / plain stores: 4096 x 4096
+        // x 1024 49 / 58 / 50, 11008 x 4096 x 512 106 / 125 / 106; fp32 NT 2048 x
+        // 2048 x 128 17.1 / 19.4 / 16.1; new buffers 65 / 57 / 61, 143 / 125 /
+        // 132). A 16-bit C is ahead either way (17-64 MB, the same C 0.73 of the
+        // MFMA layout's time with both, new ones 0.61 non-temporal, 0.67 plain),
+        // and fp32 operands are too slow for it to matter (new buffers 0.91 of the
+        // MFMA layout's time with both): plain.
         constexpr int CV = 16 / (int)sizeof(TC);             // elements of C per lane
         constexpr int STR = WT * 4 + 16;                     // padded LDS row stride
         constexpr int PROWS = WT == 128 ? 64 : WT;           // rows per pass
@@ -603,6 +612,7 @@ __global__ __launch_bounds__(256, (WT == 128 || NST == 4) ? 1 : 2) void gemm_pip
         constexpr int RPI = 64 / LPR;                        // rows per instruction
         constexpr int LB = PROWS / RPI < 16 ? PROWS / RPI : 16;
         constexpr int ROUNDS = WT / RPI / LB;
+        constexpr bool NTL = sizeof(TC) == 2 || WT == 128;   // non-temporal loads of beta's matrix
         static_assert(4 * PROWS * STR <= 2 * NST * STG * 16, "epilogue staging exceeds LDS");
         typedef TC cvec __attribute__((ext_vector_type(CV)));
         char* wl = (char*)lds + wave * (PROWS * STR);
@@ -617,7 +627,10 @@ __global__ __launch_bounds__(256, (WT == 128 || NST == 4) ? 1 : 2) void gemm_pip
 #pragma unroll
             for (int k = 0; k < LB; ++k) {
                 const int m = mrow + (rd * LB + k) * RPI;
-                if (mine(m)) o[rd & 1][k] = __builtin_nontemporal_load((const cvec*)(cil + (int64_t)m * p.epi.ldcin));
+                if (!mine(m)) continue;
+                const cvec* src = (const cvec*)(cil + (int64_t)m * p.epi.ldcin);
+                if constexpr (NTL) o[rd & 1][k] = __builtin_nontemporal_load(src);
+                else o[rd & 1][k] = *src;
             }
         };
         load_round(0);
@@ -660,7 +673,18 @@ __global__ __launch_bounds__(256, (WT == 128 || NST == 4) ? 1 : 2) void gemm_pip
                     for (int e = 0; e < 4; ++e)
                         v[4 * q + e] = (TC)(x[e] + beta * (float)o[rd & 1][k][4 * q + e] + bias[4 * q + e]);
                 }
-                __builtin_nontemporal_store(v, (cvec*)(cl + (int64_t)m * p.ldc));
+                cvec* dst = (cvec*)(cl + (int64_t)m * p.ldc);
+                if constexpr (sizeof(T) == 4) {
+                    *dst = v;
+                } else if constexpr (sizeof(TC) == 2) {
+                    __builtin_nontemporal_store(v, dst);
+                } else if (p.c_stays) {
+                    *dst = v;
+                    asm volatile("" ::: "memory");   // the two keep the compiler
+                } else {
+                    asm volatile("" ::: "memory");   // from merging the stores into a plain one
+                    __builtin_nontemporal_store(v, dst);
+                }
             }
         }
         return;
