@@ -85,3 +85,17 @@ def test_flow(ab, ct, op_a, op_b, shape, form):
             assert normwise(gb, wb) <= (BF16_BOUND if ct == "bf16" else F16_BOUND), i
     # the element in front of C
     assert np.array_equal(got.view(np.uint8).reshape(-1)[:ec], first[:ec])
+
+
+@pytest.mark.parametrize("beta,M,N,K", [(0.0, 1304, 704, 200), (1.0, 1024, 1024, 512)])
+def test_keeps_negative_zero(beta, M, N, K):
+    """no bias adds nothing, not even 0.0 to -0.0: -1 times a zero product, plus a C of -0.0"""
+    import vkblas_amd as vk
+    print(f"[case] flow -0.0 beta={beta}", flush=True)
+    a = torch.zeros(M, K, dtype=torch.float16, device="cuda:0")
+    b = torch.ones(N, K, dtype=torch.float16, device="cuda:0")
+    c = torch.full((M, N), -0.0, dtype=torch.float16, device="cuda:0")
+    vk.gemm_async(vk.DT_F16, vk.DT_F16, 0, 1, M, N, K, -1.0, a.data_ptr(), K, b.data_ptr(), K, beta, c.data_ptr(), N)
+    torch.cuda.synchronize()
+    assert vk.last_kernel() == vk.KERNEL_FLOW, vk.last_kernel()
+    assert bool((c == 0).all()) and bool(torch.signbit(c).all())

@@ -80,3 +80,19 @@ def test_add_large(K):
     got = patterns(c)
     assert np.all(np.isfinite(got))
     assert normwise(got[rows], want.reshape(M, N)[rows]) <= F16_BOUND
+
+
+@pytest.mark.parametrize("tile,ct", [(2, "f16"), (2, "f32"), (1, "f16"), (1, "f32")])
+def test_keeps_negative_zero(tile, ct):
+    """no bias adds nothing, not even 0.0 to -0.0: -1 times a zero product, plus a C of -0.0"""
+    import vkblas_amd as vk
+    print(f"[case] pipe add -0.0 tile={tile} {ct}", flush=True)
+    M, N, K = 512, 256, 256
+    a = torch.zeros(M, K, dtype=torch.float16, device="cuda:0")
+    b = torch.ones(N, K, dtype=torch.float16, device="cuda:0")
+    c = torch.full((M, N), -0.0, dtype=torch.float16 if ct == "f16" else torch.float32, device="cuda:0")
+    vk.set_override(tile, False)
+    vk.gemm_async(vk.DT_F16, ENGINE[ct], 0, 1, M, N, K, -1.0, a.data_ptr(), K, b.data_ptr(), K, 1.0, c.data_ptr(), N)
+    torch.cuda.synchronize()
+    assert vk.last_kernel() in (vk.KERNEL_PIPE256, vk.KERNEL_PIPE128, vk.KERNEL_PIPE128_4), vk.last_kernel()
+    assert bool((c == 0).all()) and bool(torch.signbit(c).all())

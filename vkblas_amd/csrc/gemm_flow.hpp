@@ -282,7 +282,8 @@ void gemm_flow_kernel(KParams p) {
     const int n = n0 + wn * WN + c;
     float bias[CV];
 #pragma unroll
-    for (int e = 0; e < CV; ++e) bias[e] = p.epi.bias && n + e < N ? bias_at(p.epi, n + e) : 0.0f;
+    for (int e = 0; e < CV; ++e)     // -0.0 where there is none: adding it changes no result's sign
+        bias[e] = p.epi.bias && n + e < N ? bias_at(p.epi, n + e) : -0.0f;
 #pragma unroll
     for (int i = 0; i < NFM; ++i) {
 #pragma unroll

@@ -636,7 +636,8 @@ __global__ __launch_bounds__(256, (WT == 128 || NST == 4) ? 1 : 2) void gemm_pip
         load_round(0);
         float bias[CV];
 #pragma unroll
-        for (int e = 0; e < CV; ++e) bias[e] = p.epi.bias ? bias_at(p.epi, n + e) : 0.0f;
+        for (int e = 0; e < CV; ++e)     // -0.0 where there is none: adding it changes no result's sign
+            bias[e] = p.epi.bias ? bias_at(p.epi, n + e) : -0.0f;
 #pragma unroll
         for (int rd = 0; rd < ROUNDS; ++rd) {
             if (rd * LB * RPI % PROWS == 0) {                // the next PROWS rows of alpha * acc
