@@ -57,6 +57,12 @@ static inline uint32_t cu_count() {
     return (uint32_t)n;
 }
 
+// Tiles as a share of the chip of cu compute units: their number per 256, on
+// which the lines below that compare it were measured.
+static inline uint64_t per_256(uint64_t tiles, uint32_t cu) {
+    return cu ? (tiles * 256 + cu - 1) / cu : tiles;
+}
+
 // Bytes of K per step of the wave-K kernel for 16-bit inputs: 128 (whole
 // 128-byte rows of a K-major operand per copy).  Measured against 64 (more
 // stages of half rows), M = N = 256, fp16, hipBLAS NN, split 4 / 16: K =
@@ -105,7 +111,8 @@ static bool flow_ok(const vkb_gemm_args* a, const KParams& p) {
            span_a < (1ull << 31) && span_b < (1ull << 31);
 }
 
-// gemm_flow_kernel's form, from the number of 128 x 128 tiles t (one box, fp16 us):
+// gemm_flow_kernel's form, from the number of 128 x 128 tiles t per 256 CUs (one box,
+// fp16 us):
 //  * N of one 64-column tile, or t at most half the CUs: 128 x 64 tiles, three
 //    stages, two workgroups per CU (1000^3, t = 64, 11.2 against 13.8 on 128 x 128;
 //    1280 x 1280 x 1000, 100, 11.2 / 13.7; 1536 x 1536 x 1000, 144, 15.9 / 13.5);
@@ -116,12 +123,12 @@ static bool flow_ok(const vkb_gemm_args* a, const KParams& p) {
 //    K of a single step: one stage and three or four workgroups per CU (64 x 1024 x
 //    1024 x 64 29.7 against 34.7 with two stages).
 template <typename T, typename TC>
-static int launch_flow(const vkb_gemm_args* a, KParams p, bool ak, bool bk, hipStream_t st) {
+static int launch_flow(const vkb_gemm_args* a, KParams p, bool ak, bool bk, uint32_t cu, hipStream_t st) {
     if constexpr (sizeof(T) == 2) {
         const uint64_t mats = (uint64_t)p.batch * p.split;
         p.tiles_m = (a->M + 127) / 128;
         p.tiles_n = (a->N + 127) / 128;
-        const uint64_t t = (uint64_t)p.tiles_m * p.tiles_n * mats;
+        const uint64_t t = per_256((uint64_t)p.tiles_m * p.tiles_n * mats, cu);
         const bool narrow = a->N <= 64 || t <= 128;
         if (narrow) p.tiles_n = (a->N + 63) / 64;
         const uint64_t grid = (uint64_t)p.tiles_m * p.tiles_n * mats;
@@ -149,7 +156,7 @@ static int launch_flow(const vkb_gemm_args* a, KParams p, bool ak, bool bk, hipS
 // tile in its dimension; a tile's rows must span less than 2^31 bytes) or the
 // launch: the larger tiles of the generic kernel then may.
 template <typename T>
-static uint32_t direct_tile(const vkb_gemm_args* a, uint64_t mats) {
+static uint32_t direct_tile(const vkb_gemm_args* a, uint64_t mats, uint32_t cu) {
     auto tiles = [&](uint32_t tm, uint32_t tn) {
         return (uint64_t)((a->M + tm - 1) / tm) * ((a->N + tn - 1) / tn) * mats;
     };
@@ -162,8 +169,8 @@ static uint32_t direct_tile(const vkb_gemm_args* a, uint64_t mats) {
                (ra * (uint64_t)a->lda + 64) * sizeof(T) < (1ull << 31) &&
                (rb * (uint64_t)a->ldb + 64) * sizeof(T) < (1ull << 31);
     };
-    if (tiles(64, 64) >= 144 && fits(64, 64)) return 64;
-    if ((sizeof(T) == 2 || tiles(32, 32) >= 128) && fits(32, 32)) return 32;
+    if (per_256(tiles(64, 64), cu) >= 144 && fits(64, 64)) return 64;
+    if ((sizeof(T) == 2 || per_256(tiles(32, 32), cu) >= 128) && fits(32, 32)) return 32;
     if (sizeof(T) == 4 && fits(16, 32)) return 16;
     return 0;
 }
@@ -339,22 +346,24 @@ static int launch_gemm_typed(const vkb_gemm_args* a, int tile, hipStream_t st) {
         if (a->direct && !p.ptr_array && !a->generic_only &&
             (tile == VKB_TILE_64 || tile == VKB_TILE_128 || tile == VKB_TILE_256) &&
             !(tile == VKB_TILE_64 && p.split > 1 && full)) {
+            const uint32_t cu = cu_count();
             const uint64_t mats = (uint64_t)p.batch * p.split;
-            const uint64_t t64 = (uint64_t)((a->M + 63) / 64) * ((a->N + 63) / 64) * mats;
+            const uint64_t t64 = per_256((uint64_t)((a->M + 63) / 64) * ((a->N + 63) / 64) * mats, cu);
             const bool pipe = pipe_ok && tile != VKB_TILE_64;
-            const bool add = pipe && tile == VKB_TILE_128 && p.split == 1 && grid <= 256 &&
+            const bool add = pipe && tile == VKB_TILE_128 && p.split == 1 && per_256(grid, cu) <= 256 &&
                              a->scalar_mode == VKB_SCALAR_HOST && a->beta != 0.0f && a->K <= 1024;
             if (a->direct == 1 && ((!pipe && t64 >= 144) || add) && flow_ok<T>(a, p)) {
                 report(VKB_KERN_FLOW);
-                return launch_flow<T, TC>(a, p, ak, bk, st);
+                return launch_flow<T, TC>(a, p, ak, bk, cu, st);
             }
             const uint32_t klen = p.split > 1 ? p.kps : a->K;
             const bool want = a->direct == 2 ? true
-                            : pipe ? sizeof(T) == 4 && tile == VKB_TILE_128 && p.split == 1 && grid <= 128
+                            : pipe ? sizeof(T) == 4 && tile == VKB_TILE_128 && p.split == 1 &&
+                                   per_256(grid, cu) <= 128
                             : full ? t64 < (ak && bk ? (sizeof(T) == 4 ? 144u : 96u) : klen * sizeof(T) >= 512 ? 192u : 144u)
                                    : !direct_loses<T>(ak, bk, t64, klen) &&
                                          ((uint64_t)klen * sizeof(T) >= 512 || t64 <= 256);
-            const uint32_t dt = want ? direct_tile<T>(a, mats) : 0;
+            const uint32_t dt = want ? direct_tile<T>(a, mats, cu) : 0;
             if (dt) {
                 report(VKB_KERN_DIRECT);
                 return launch_direct<T, TC>(a, p, dt, ak, bk, st);
