@@ -3,7 +3,8 @@ edges of its tiles: one past and one short of a tile, one k, K around its K
 step (16 fp32, 32 16-bit) and around a whole round of loads in flight, every
 layout and type pair, odd leading dimensions with NaN in the padding,
 operands one element off any alignment, batches, beta with C in place or
-apart, a bias; against the CPU oracle.  C's padding must come back untouched."""
+apart, a bias; against the CPU oracle.  C's padding must come back untouched.  Split-K
+pass 1 with a ragged last slice."""
 import numpy as np
 import pytest
 import torch
@@ -23,7 +24,7 @@ SHAPES = [(33, 32, 1, 1), (65, 47, 15, 1), (95, 33, 33, 2), (129, 65, 64, 3),   
           (65, 64, 257, 72), (129, 127, 511, 36), (193, 321, 1027, 7)]           # 64 x 64
 
 
-@pytest.mark.parametrize("form", ["plain", "apart"])
+@pytest.mark.parametrize("form", ["plain", "apart", "in_place"])
 @pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
 @pytest.mark.parametrize("op_a,op_b", [(0, 0), (0, 1), (1, 0), (1, 1)])
 @pytest.mark.parametrize("ab,ct", TYPES)
@@ -76,6 +77,33 @@ def test_direct(ab, ct, op_a, op_b, shape, form):
         assert np.array_equal(g[:, N:], w[:, N:]), "C padding written"
         assert np.all(np.isfinite(g[:, :N]))
         assert normwise(g[:, :N], w[:, :N]) <= bound, i
+
+
+@pytest.mark.parametrize("form", ["plain", "in_place"])
+@pytest.mark.parametrize("M,N,K,split", [(33, 35, 1000, 3), (97, 65, 2003, 4), (193, 129, 777, 2)])
+@pytest.mark.parametrize("op_a,op_b", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("ab,ct", [("f32", "f32"), ("f16", "f16"), ("bf16", "f32")])
+def test_direct_split(ab, ct, op_a, op_b, M, N, K, split, form):
+    """pass 1 of a caller's split: slices that start past k 0, the last one shorter"""
+    import vkblas_amd as vk
+    print(f"[case] direct split {ab}>{ct} op={op_a}{op_b} {M}x{N}x{K}/{split} {form}", flush=True)
+    r = np.random.default_rng(M + 3 * N + 7 * K)
+    ra, lda = (K, M) if op_a else (M, K)
+    rb, ldb = (N, K) if op_b else (K, N)
+    a, b, c = (CONV[t](r.uniform(-1, 1, 1 + n).astype(np.float32))
+               for t, n in ((ab, ra * lda), (ab, rb * ldb), (ct, M * N)))
+    beta = 0.0 if form == "plain" else -0.5
+    want = c[1:].copy()
+    oracle.ref_gemm_epi_rm(ab, ct, op_a, op_b, M, N, K, a[1:].copy(), lda, b[1:].copy(), ldb, 1.25, beta, want.copy(),
+                           N, want, N, None)
+    dA, dB, dC = _dev(a, ab), _dev(b, ab), _dev(c, ct)
+    vk.gemm_async(ENGINE[ab], ENGINE[ct], op_a, op_b, M, N, K, 1.25, dA.data_ptr() + dA.element_size(), lda,
+                  dB.data_ptr() + dB.element_size(), ldb, beta, dC.data_ptr() + dC.element_size(), N, split_k=split)
+    assert (vk.last_path(), vk.last_kernel()) == (vk.PATH_SPLITK, vk.KERNEL_DIRECT), vk.last_kernel()
+    got = patterns(dC)
+    assert got[0] == c[0], "the element in front of C written"
+    bound = BF16_BOUND if ct == "bf16" else f32_bound(K) if ab == "f32" else F16_BOUND
+    assert normwise(BACK[ct](got[1:].copy()), BACK[ct](want)) <= bound
 
 
 # type, op_a, op_b, M, N, K, batch, kernel: both sides of the lines in tiles of 64 x 64

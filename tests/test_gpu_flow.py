@@ -3,7 +3,8 @@ tiles and forms: K of one step, one short of and one past it in 16-byte chunks,
 past its stages; M and N one past and one short of a tile where the layout takes
 them; the form for few, for one wave of and for many tiles; NaN in the padding of
 every operand, C without any alignment, beta with C in place or apart, a bias;
-against the CPU oracle.  C's padding must come back untouched."""
+against the CPU oracle.  C's padding must come back untouched.  Split-K pass 1 with a
+ragged last slice, and the calls that add to C instead of the pipelined kernel."""
 import numpy as np
 import pytest
 import torch
@@ -18,11 +19,12 @@ pytestmark = pytest.mark.gpu
 # K to one of 8 unless both are MN-major):
 SHAPES = [(257, 63, 65, 40), (129, 127, 191, 40),      # 128 x 64 tiles: N of one, few of 128 x 128
           (641, 1153, 328, 4),                         # 128 x 128, three stages, eight waves (240 tiles)
+          (1301, 703, 40, 1), (1601, 1537, 64, 1),     # three stages, one step: 128 x 64, eight waves
           (129, 129, 57, 96),                          # one stage (384 tiles, a single partial step)
           (257, 255, 72, 72), (130, 257, 200, 50)]     # two stages
 
 
-@pytest.mark.parametrize("form", ["plain", "apart"])
+@pytest.mark.parametrize("form", ["plain", "apart", "in_place"])
 @pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
 @pytest.mark.parametrize("op_a,op_b", [(0, 0), (0, 1), (1, 0), (1, 1)])
 @pytest.mark.parametrize("ab,ct", [("f16", "f16"), ("f16", "f32"), ("bf16", "bf16"), ("bf16", "f32")])
@@ -85,6 +87,46 @@ def test_flow(ab, ct, op_a, op_b, shape, form):
             assert normwise(gb, wb) <= (BF16_BOUND if ct == "bf16" else F16_BOUND), i
     # the element in front of C
     assert np.array_equal(got.view(np.uint8).reshape(-1)[:ec], first[:ec])
+
+
+@pytest.mark.parametrize("form", ["plain", "in_place"])
+@pytest.mark.parametrize("M,N,K,split", [(520, 520, 600, 3), (1032, 264, 2056, 4)])
+@pytest.mark.parametrize("op_a,op_b", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("ab,ct", [("f16", "f16"), ("bf16", "f32")])
+def test_flow_split(ab, ct, op_a, op_b, M, N, K, split, form):
+    """pass 1 of a caller's split: slices that start past k 0, the last one shorter"""
+    import vkblas_amd as vk
+    print(f"[case] flow split {ab}>{ct} op={op_a}{op_b} {M}x{N}x{K}/{split} {form}", flush=True)
+    _adds(vk, ab, ct, op_a, op_b, M, N, K, 0.0 if form == "plain" else -0.5, split, vk.PATH_SPLITK, vk.KERNEL_FLOW)
+
+
+@pytest.mark.parametrize("M,N,K,beta,kernel", [
+    (1024, 1024, 512, -0.5, "FLOW"), (256, 4096, 1024, 1.0, "FLOW"), (200, 8192, 128, 1.0, "FLOW"),
+    (1024, 1024, 512, 0.0, "PIPE128_4"), (256, 4096, 1152, 1.0, "PIPE128_4")])
+@pytest.mark.parametrize("ab,ct", [("f16", "f16"), ("bf16", "f32")])
+@pytest.mark.parametrize("op_a,op_b", [(0, 1), (1, 0)])
+def test_adds_to_c(op_a, op_b, ab, ct, M, N, K, beta, kernel):
+    """one wave of 128 x 128 tiles: this kernel where beta adds to C in place after at most
+    1024 k, else the pipelined one"""
+    import vkblas_amd as vk
+    print(f"[case] adds {ab}>{ct} op={op_a}{op_b} {M}x{N}x{K} beta={beta}", flush=True)
+    _adds(vk, ab, ct, op_a, op_b, M, N, K, beta, 0, vk.PATH_TILE128, getattr(vk, "KERNEL_" + kernel))
+
+
+def _adds(vk, ab, ct, op_a, op_b, M, N, K, beta, split, path, kernel):
+    r = np.random.default_rng(M + 3 * N + 7 * K)
+    lda, ldb = (M if op_a else K), (K if op_b else N)
+    a, b, c = (CONV[t](r.uniform(-1, 1, n).astype(np.float32)) for t, n in ((ab, M * K), (ab, N * K), (ct, M * N)))
+    rows = oracle.sample_rows(M, 16)
+    want = c.copy()
+    oracle.ref_gemm_epi_rm(ab, ct, op_a, op_b, M, N, K, a, lda, b, ldb, 1.25, beta, c, N, want, N, None, rows=rows)
+    dA, dB, dC = _dev(a, ab), _dev(b, ab), _dev(c, ct)
+    vk.gemm_async(ENGINE[ab], ENGINE[ct], op_a, op_b, M, N, K, 1.25, dA.data_ptr(), lda, dB.data_ptr(), ldb, beta,
+                  dC.data_ptr(), N, split_k=split)
+    assert (vk.last_path(), vk.last_kernel()) == (path, kernel), (vk.last_path(), vk.last_kernel())
+    got = BACK[ct](patterns(dC)).reshape(M, N)
+    assert np.all(np.isfinite(got))
+    assert normwise(got[rows], BACK[ct](want).reshape(M, N)[rows]) <= (BF16_BOUND if ct == "bf16" else F16_BOUND)
 
 
 @pytest.mark.parametrize("beta,M,N,K", [(0.0, 1304, 704, 200), (1.0, 1024, 1024, 512)])

@@ -60,7 +60,8 @@ def kernels(tmp_path_factory):
 def test_every_kernel_family_is_present(kernels):
     names = " ".join(k[0] for k in kernels)
     for fam in ("gemm_pipe_kernel", "gemm_wavek_kernel", "gemm_kernel", "splitk_reduce_kernel", "gemv_kernel",
-                "skinny_lds_kernel", "decode_lds_kernel", "skinny_n_kernel", "skinny_nh_kernel"):
+                "skinny_lds_kernel", "decode_lds_kernel", "skinny_n_kernel", "skinny_nh_kernel", "gemm_direct_kernel",
+                "gemm_flow_kernel"):
         assert fam in names, fam
 
 
