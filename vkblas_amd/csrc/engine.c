@@ -782,8 +782,11 @@ static vkblas_status_t gemm_impl(vkblas_dtype_t ab_type, vkblas_dtype_t c_type, 
      * (VKB_TILE_64Q) then the parts' sums, VKB_WAVEK_NQ x the partials */
     const int direct = plan.path == VKBLAS_PATH_SKINNY && small_decode(ab_type, op_b, M, N, K, lda, ldb);
     if (direct && plan.split > 1 && !ws_ext) {
-        /* a decode plan with a K split is refused under stream capture
-         * whatever kernel would run it, as ws_acquire refuses it */
+        /* Under stream capture a decode plan with a K split has always been
+         * refused (for its partials), and a caller has to know from the plan
+         * whether a call can be captured: so also where the kernel chosen
+         * needs no partials.  With the no-alloc entry point such a plan always
+         * runs: its partials are at most 4.1 MiB of the scratch's 64. */
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(hs, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return VKBLAS_ERR_INIT;
     }

@@ -44,7 +44,7 @@ constexpr int flow_wg_per_cu(int BN, int NST, bool kmajor) {
     return NST == 1 ? (kmajor ? 4 : 3) : NST * (128 + BN) * 128 > 80 * 1024 ? 1 : 2;
 }
 // EARLY: beta's matrix is read before the K loop, which then hides its latency
-// (bf16 -> fp32 TN 4096 x 1024 x 512, beta = 1: 14.5 -> 11.0 us); a form of its own,
+// (bf16 -> fp32 TN 4096 x 1024 x 512, beta = 1: 14.5 -> 12.5 us); a form of its own,
 // as its registers and the early scalars cost the others 3 % (attention bf16).
 template <typename T, typename TC, bool AK, bool BKM, int BN, int NST, int WAVES, bool EARLY = false>
 __global__ __launch_bounds__(64 * WAVES, flow_wg_per_cu(BN, NST, AK && BKM) * WAVES / 4)

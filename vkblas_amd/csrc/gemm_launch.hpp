@@ -251,12 +251,9 @@ static int launch_gemm_typed(const vkb_gemm_args* a, int tile, hipStream_t st) {
         return (int)hipErrorInvalidValue;
     const bool multi = p.batch > 1;
     if (p.ptr_array) {
-        // the matrices' alignment is checked per batch in the kernel, which
-        // always runs the checked instantiation (no pipelined kernel)
+        // the matrices' alignment is not known here: always the checked
+        // instantiation, which takes any
         if (p.split > 1) return (int)hipErrorInvalidValue;
-        p.vec_a = a->lda % VEC == 0;
-        p.vec_b = a->ldb % VEC == 0;
-        p.vec_c = a->ldc % 4 == 0;
     } else {
         p.vec_a = (a->lda % VEC == 0) && aligned(a->A, 16) && (!multi || a->stride_a % VEC == 0);
         p.vec_b = (a->ldb % VEC == 0) && aligned(a->B, 16) && (!multi || a->stride_b % VEC == 0);

@@ -66,8 +66,7 @@ struct KParams {
     // Cin (beta's matrix) and the bias vector; vec_c covers Cin's alignment too
     EpiParams epi;
     // A, B, C are device arrays of `batch` matrix pointers (the sa / sb / sc
-    // strides are unused); vec_* then also need each matrix aligned, which
-    // the kernel checks per batch
+    // strides are unused), of any element alignment
     int ptr_array;
     // wave-K split-K pass 1 with each K slice over nq workgroups (nq > 1):
     // their sums in qpart, their arrival counters in qcnt
