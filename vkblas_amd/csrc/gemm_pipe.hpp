@@ -604,7 +604,9 @@ __global__ __launch_bounds__(256, (WT == 128 || NST == 4) ? 1 : 2) void gemm_pip
         // 132). A 16-bit C is ahead either way (17-64 MB, the same C 0.73 of the
         // MFMA layout's time with both, new ones 0.61 non-temporal, 0.67 plain),
         // and fp32 operands are too slow for it to matter (new buffers 0.91 of the
-        // MFMA layout's time with both): plain.
+        // MFMA layout's time with both): plain, and on 128 x 128 tiles too, whose C
+        // is small against such operands, and where the choice alone cost the
+        // kernel's other calls 1 % (256 x 256 x 65536 with its reduce 19.3 / 19.5).
         constexpr int CV = 16 / (int)sizeof(TC);             // elements of C per lane
         constexpr int STR = WT * 4 + 16;                     // padded LDS row stride
         constexpr int PROWS = WT == 128 ? 64 : WT;           // rows per pass
@@ -675,7 +677,7 @@ __global__ __launch_bounds__(256, (WT == 128 || NST == 4) ? 1 : 2) void gemm_pip
                         v[4 * q + e] = (TC)(x[e] + beta * (float)o[rd & 1][k][4 * q + e] + bias[4 * q + e]);
                 }
                 cvec* dst = (cvec*)(cl + (int64_t)m * p.ldc);
-                if constexpr (sizeof(T) == 4) {
+                if constexpr (sizeof(TC) == 4 && (sizeof(T) == 4 || WT == 64)) {
                     *dst = v;
                 } else if constexpr (sizeof(TC) == 2) {
                     __builtin_nontemporal_store(v, dst);
